@@ -1,33 +1,48 @@
 // Prefill on the matrix cores in the canonical order: bit-exact.
 //
-// gemm_exact — v_mfma_f32_32x32x1_2b_f32 (K = 1, two 32 x 32 blocks) rounds
-// each element once, as a fused multiply-add: d = c + a b is fmaf(a, b, c)
-// bit for bit (checked on the GPU by harness.hip's mfma_fma_check over
-// random, cancelling, halfway, denormal, overflowing, infinite and NaN
-// operands). So a range's chain s = fma(w_k, x_k, s), in k order from +0
-// (matmul.wgsl:121-126, 224-230), runs as a chain of these instructions, one
-// k at a time, for 2,048 outputs at once; a range's sums then add into the
-// totals in order on the VALU (matmul.wgsl:134-137), as gemm_canonical adds
-// them. Every output is gemm_canonical's bits, and decode's.
+// gemm_exact — v_mfma_f32_32x32x2_f32 (K = 2, one 32 x 32 block) adds its two
+// products one after the other, each as a fused multiply-add: d = fmaf(a1,
+// b1, fmaf(a0, b0, c)) bit for bit (checked on the GPU by harness.hip's
+// mfma_chain_check over random, cancelling, halfway, denormal, overflowing,
+// infinite and NaN operands). So a range's chain s = fma(w_k, x_k, s), in k
+// order from +0 (matmul.wgsl:121-126, 224-230), runs as a chain of these
+// instructions, two ks at a time, for 1,024 outputs at once; a range's sums
+// then add into the totals in order on the VALU (matmul.wgsl:134-137), as
+// gemm_canonical adds them. Every output is gemm_canonical's bits, and
+// decode's.
 //
-// A wave takes 64 rows x TT tokens. At each k lane l supplies row R + l's
-// weight as the A operand (lanes 0-31 block 0's rows, 32-63 block 1's).
-// TT = 64: lane l supplies token T + l's input as B (lanes 0-31 block 0's
-// columns, 32-63 block 1's), and two instructions a k, each broadcasting one
-// block's A to both blocks (CBSZ 1, ABID 0 and 1), give rows R .. R + 31 and
-// R + 32 .. R + 63 against tokens T .. T + 63. TT = 32 (for steps too small
-// to give every SIMD two waves of 64 x 64): lanes l and l + 32 both supply
-// token T + l % 32, and one instruction a k gives rows R .. R + 63 against
-// tokens T .. T + 31. Each lane decodes its row's group (32 exact f32 weights) and
-// loads its token's 32 inputs into registers, a group ahead; nothing goes
-// through LDS and the waves of a workgroup never wait for one another. The
-// VALU's share — a group's decode, a range's adds — is small beside the 64
-// matrix instructions a group, and runs while they do.
+// What bounds it: the f32 matrix instructions and the VALU take turns on a
+// SIMD — an instruction of the one adds its whole time to the other's (a
+// probe of four independent products and n VALU instructions a wave, at one
+// and two waves a SIMD: 72 cycles a product alone, + 4.4 a v_perm_b32 or
+// v_fma_mix_f32, + 2.7 a v_add_f32 past the second) — so beside the products
+// (64 cycles each, 98% of the FP32 peak where the K = 1 shape sustains 88%)
+// the time is the VALU work a product, and the design is what keeps that
+// small. The operands of ks 2m and 2m + 1 are one register whose lower
+// half-wave holds k 2m and whose upper k 2m + 1: each lane decodes its own
+// half of its row's weights (Half below: 32 instructions a Q4_0 group), and
+// the inputs lie in LDS split into even and odd ks, so they are read as
+// operands with no instruction between. A 32-row group and 64 tokens take 32
+// products and about 40 VALU instructions, 32 more at a range's end.
 //
-// Result layout of one instruction (register v of 32, lane l): block v / 16,
-// in it column l % 32 and row 8 ((v % 16) / 4) + 4 (l / 32) + v % 4 — rows
-// p, p + 1 (p even) in one lane, so a gated product's gate and up totals
-// (rows 2r, 2r + 1) meet there.
+// A workgroup takes 256 rows x TB x 32 tokens, eight waves of 32 rows each
+// sharing its inputs: each group's are copied once, eight lanes a token's
+// 128-byte line (a lane a token touches 64 lines a load, eight times over:
+// with the loads spread among the products a line was fetched again for
+// each), through registers into a ring of LDS stages, two groups between the
+// workgroup's meetings (four: 144 against 142 us at 2,048 x 2,048 x 2,048,
+// and a workgroup a CU less). Reading the inputs a slot ahead of their
+// products, or spreading the decode among them by hand, measured no better:
+// the SIMD's other waves cover the waits. Measured (Q4_0, two sides A/B):
+// against the K = 1 form, 64 x 64 a wave with both operands in registers,
+// 2,048 tokens through Llama 3.2 1B's layer 2,075 -> 1,968 us (120 -> 127
+// TFLOP/s), 4,096 x 1,024 x 512 57 -> 46, 2 x 3,072 x 1,024 x 512 gated 100
+// -> 81, 4,096 x 1,152 x 2,048 BF16 181 -> 158, 8,192 x 2,048 x 300 F32 276 ->
+// 153 us.
+//
+// Result layout of the instruction (register v of 16, lane l): column l % 32,
+// row 8 (v / 4) + 4 (l / 32) + v % 4 — rows p, p + 1 (p even) in one lane, so
+// a gated product's gate and up totals (rows 2r, 2r + 1) meet there.
 #include "decode.hpp"
 #include "plan.hpp"
 #include "product.hpp"
@@ -40,8 +55,8 @@ namespace {
 typedef float f32x32 __attribute__((ext_vector_type(32)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr uint32_t kWaveRows = 64;   // rows a wave
-constexpr uint32_t kWaves = 4;       // waves a workgroup, each its own 64 rows
+constexpr uint32_t kWaveRows = 32;   // rows a wave
+constexpr uint32_t kWaves = 8;       // waves a workgroup, each its own 32 rows
 
 // Four weights from four code bytes as the decodes' chain4 makes them: two
 // codes a v_perm_b32 as binary16 1024 + b, then one v_fma_mix_f32 a weight,
@@ -57,7 +72,7 @@ __device__ __forceinline__ void weights4(uint32_t codes, float scale, float offs
 // The 32 exact weights of a group as loaded: the values of formats.hpp's
 // weight(), which the VALU tile stages. Q4_0, Q8_0 and Q6_K by the lift of
 // decode.hpp's chain_q4_0, chain_q8_0 and chain_q6_k (1.75 instructions a
-// weight against weight()'s 3: C4 105 -> 111 TFLOP/s), the others by weight().
+// weight against weight()'s 3), the others by weight(). The short-step tiles'.
 template <uint32_t F>
 __device__ __forceinline__ void weights_of(const Raw<F>& r, float* w) {
     if constexpr (F == kQ4_0) {
@@ -108,6 +123,195 @@ __device__ __forceinline__ void weights_of(const Raw<F>& r, float* w) {
     }
 }
 
+// The upper half-wave of `a` against the lower of `b`: afterwards a holds the
+// two lower halves (a's, then b's), b the two upper ones.
+__device__ __forceinline__ void swap32(float& a, float& b) {
+    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    const uint32_t s0 = s[0], s1 = s[1];
+    a = __uint_as_float(s0), b = __uint_as_float(s1);
+}
+
+// A lane's share of one row's group for the K = 2 instruction: lane half h
+// (lanes 0-31: 0) takes ks h, h + 2, ..., its sixteen weights w of weights_of.
+// decode(r, h) works out what the whole group shares; four(j, w) gives ks
+// 8j + h, 8j + 2 + h, 8j + 4 + h, 8j + 6 + h. Each lane makes its own half's
+// weights alone, so the two lanes of a row do a group's decode between them.
+template <uint32_t F>
+struct Half;
+
+// Q4_0: a code dword shifted by 8h holds its lane's codes in bytes 0 and 2;
+// under 0x54 a half is 64 + m / 16 for its low byte m (chain_q4_0_wide), so
+// a mask-and-or makes two of them: (64 + l / 16) 16d - 1032d = (l - 8) d and
+// (64 + h) d - 72 d = (h - 8) d, exact. 1.75 instructions a weight.
+template <>
+struct Half<kQ4_0> {
+    uint32_t w[4];
+    float d, low, d16, high;
+    __device__ __forceinline__ void decode(const Raw<kQ4_0>& r, uint32_t h) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[i] = r.w[i] >> (8 * h);
+        d = half_to_float(r.d);
+        d16 = 16.0f * d, low = -1032.0f * d, high = -72.0f * d;
+    }
+    __device__ __forceinline__ void four(int j, float* o) const {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const bool nib = j >= 2;
+            const uint32_t c = w[2 * (j & 1) + i];
+            const half2_t u = __builtin_bit_cast(
+                half2_t, nib ? and_or(c, 0x00F000F0u, 0x54005400u) : and_or(c, 0x000F000Fu, 0x54005400u));
+            o[2 * i] = __builtin_fmaf(static_cast<float>(u.x), nib ? d : d16, nib ? high : low);
+            o[2 * i + 1] = __builtin_fmaf(static_cast<float>(u.y), nib ? d : d16, nib ? high : low);
+        }
+    }
+};
+
+// Q4_1: the codes as halves 1024 + q less 1024 (high nibbles 16 q, against
+// d / 16: the same product), then fma(q, d, m) — weight()'s one rounding.
+template <>
+struct Half<kQ4_1> {
+    uint32_t w[4];
+    float d, m, d16;
+    __device__ __forceinline__ void decode(const Raw<kQ4_1>& r, uint32_t h) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[i] = r.w[i] >> (8 * h);
+        d = half_to_float(r.dm & 0xFFFFu), m = half_to_float(r.dm >> 16);
+        d16 = d * 0.0625f;
+    }
+    __device__ __forceinline__ void four(int j, float* o) const {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const bool nib = j >= 2;
+            const uint32_t c = w[2 * (j & 1) + i];
+            const half2_t base = {1024.0f16, 1024.0f16};
+            const half2_t u = __builtin_bit_cast(half2_t, nib ? and_or(c, 0x00F000F0u, 0x64006400u)
+                                                              : and_or(c, 0x000F000Fu, 0x64006400u)) -
+                              base;
+            o[2 * i] = __builtin_fmaf(static_cast<float>(u.x), nib ? d16 : d, m);
+            o[2 * i + 1] = __builtin_fmaf(static_cast<float>(u.y), nib ? d16 : d, m);
+        }
+    }
+};
+
+// Two code bytes of a dword, h and h + 2, lifted to binary16 1024 + b.
+__device__ __forceinline__ uint32_t half_selector(uint32_t h) { return h ? 0x04030401u : 0x04020400u; }
+
+template <>
+struct Half<kQ8_0> {
+    uint32_t w[8], selector;
+    float d, offset;
+    __device__ __forceinline__ void decode(const Raw<kQ8_0>& r, uint32_t h) {
+        selector = half_selector(h);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[i] = r.w[i];
+        d = half_to_float(r.d), offset = -1152.0f * d;
+    }
+    __device__ __forceinline__ void four(int j, float* o) const {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const half2_t u = lift(w[2 * j + i] ^ 0x80808080u, selector);
+            o[2 * i] = __builtin_fmaf(static_cast<float>(u.x), d, offset);
+            o[2 * i + 1] = __builtin_fmaf(static_cast<float>(u.y), d, offset);
+        }
+    }
+};
+
+// Q6_K: the 6-bit codes assembled as chain_q6_k assembles them.
+template <>
+struct Half<kQ6_K> {
+    uint32_t lo[4], a[2], b[2], selector;
+    float first, first_offset, second, second_offset;
+    __device__ __forceinline__ void decode(const Raw<kQ6_K>& r, uint32_t h) {
+        selector = half_selector(h);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) lo[i] = r.lo[i];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) a[i] = r.hi[i] & 0x33333333u, b[i] = (r.hi[i] >> 2) & 0x33333333u;
+        const float d = half_to_float(r.d);
+        first = d * static_cast<float>(static_cast<int8_t>(r.sc & 0xFFu));
+        second = d * static_cast<float>(static_cast<int8_t>((r.sc >> 8) & 0xFFu));
+        first_offset = -1056.0f * first, second_offset = -1056.0f * second;
+    }
+    __device__ __forceinline__ void four(int j, float* o) const {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t pairs = (j & 1) ? b[i] : a[i];  // weights 8j .. 8j + 7: pairs at bits 2j
+            const uint32_t l = lo[2 * (j & 1) + i];
+            const half2_t u = lift(j < 2 ? bitfield_insert(0x0F0F0F0Fu, l, pairs << 4)
+                                         : bitfield_insert(0x0F0F0F0Fu, l >> 4, pairs),
+                                   selector);
+            const float scale = j < 2 ? first : second, offset = j < 2 ? first_offset : second_offset;
+            o[2 * i] = __builtin_fmaf(static_cast<float>(u.x), scale, offset);
+            o[2 * i + 1] = __builtin_fmaf(static_cast<float>(u.y), scale, offset);
+        }
+    }
+};
+
+// The plain formats: the lower half-wave loads ks 0 .. 15 of its row, the
+// upper 16 .. 31; swapping two neighbours between the halves gives one
+// register of ks 2m, 2m + 1 and one of ks 16 + 2m, 17 + 2m, as the halves
+// take them.
+template <uint32_t F>
+struct HalfRaw : Raw<F> {
+    __device__ __forceinline__ void load_half(const uint8_t* piece, uint64_t blocks, uint64_t gi, uint32_t) {
+        this->load(piece, blocks, gi);
+    }
+};
+template <uint32_t F>
+struct PlainHalfRaw {
+    static constexpr int kWords = F == kF32 ? 16 : 8;
+    uint32_t w[kWords];
+    __device__ __forceinline__ void load_half(const uint8_t* piece, uint64_t, uint64_t gi, uint32_t h) {
+        const uint4* at = reinterpret_cast<const uint4*>(piece + 8 * kWords * gi + 4 * kWords * h);
+#pragma unroll
+        for (int v = 0; v < kWords / 4; ++v) {
+            const uint4 q = at[v];
+            w[4 * v] = q.x, w[4 * v + 1] = q.y, w[4 * v + 2] = q.z, w[4 * v + 3] = q.w;
+        }
+    }
+};
+template <>
+struct HalfRaw<kF32> : PlainHalfRaw<kF32> {};
+template <>
+struct HalfRaw<kF16> : PlainHalfRaw<kF16> {};
+template <>
+struct HalfRaw<kBF16> : PlainHalfRaw<kBF16> {};
+
+template <uint32_t F>
+struct PlainHalf {
+    float w[16];
+    __device__ __forceinline__ void decode(const HalfRaw<F>& r, uint32_t) {
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+            float e, o;
+            if constexpr (F == kF32) {
+                e = __uint_as_float(r.w[2 * m]), o = __uint_as_float(r.w[2 * m + 1]);
+            } else {
+                e = F == kF16 ? half_to_float(r.w[m] & 0xFFFFu) : bf16_low(r.w[m]);
+                o = F == kF16 ? half_to_float(r.w[m] >> 16) : bf16_high(r.w[m]);
+            }
+            swap32(e, o);
+            w[m] = e, w[8 + m] = o;
+        }
+    }
+    __device__ __forceinline__ void four(int j, float* o) const {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = w[4 * j + i];
+    }
+};
+template <>
+struct Half<kF32> : PlainHalf<kF32> {};
+template <>
+struct Half<kF16> : PlainHalf<kF16> {};
+template <>
+struct Half<kBF16> : PlainHalf<kBF16> {};
+
+// A wave's range sums: 32 rows by TB token blocks of 32.
+template <int TB>
+struct Sums {
+    f32x16 v[TB];
+};
+
 // SPLIT (the split along K, matmul.wgsl:592-695): `chunks` workgroups a tile,
 // chunk c taking ranges [32c / chunks, 32(c + 1) / chunks) and writing each
 // range's sum to range_sums ([32][tokens][rows], range first) instead of
@@ -116,180 +320,204 @@ __device__ __forceinline__ void weights_of(const Raw<F>& r, float* w) {
 // `quads`: rows a multiple of 4 and range_sums 16-byte aligned, so a lane's
 // four registers of consecutive rows go out as one 16-byte store (C6's split
 // 20.9 -> 18.3 us against a store a register).
-template <uint32_t F, uint32_t TT, bool FULL, bool CLIP, bool SPLIT = false>
-__global__ __launch_bounds__(256, 2) void gemm_exact(Product a, uint32_t token_tiles, uint32_t row_tiles,
-                                                     uint32_t chunks, float* range_sums, bool quads) {
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    const uint32_t tile_t = blockIdx.x % token_tiles, tile_r = (blockIdx.x / token_tiles) % row_tiles;
-    const uint32_t chunk = blockIdx.x / (token_tiles * row_tiles);
-    const uint32_t T = tile_t * TT, R = (tile_r * kWaves + wave) * kWaveRows;
-    if (R >= a.rows) return;  // the whole wave: no barrier follows
+template <int TB>
+__device__ __forceinline__ void store_sums(const Product& a, const Sums<TB>& s, uint32_t range, uint32_t R, uint32_t T,
+                                           float* range_sums, bool quads) {
+    const uint32_t lane = threadIdx.x & 63u;
+#pragma unroll
+    for (int tb = 0; tb < TB; ++tb) {
+        const uint32_t token = T + 32 * tb + (lane & 31u);
+        if (token >= a.tokens) continue;
+        float* const row = range_sums + (static_cast<uint64_t>(range) * a.tokens + token) * a.rows;
+#pragma unroll
+        for (int v = 0; v < 16; v += 4) {
+            const uint32_t p = R + 2 * v + 4 * (lane >> 5);
+            const float q[4] = {s.v[tb][v], s.v[tb][v + 1], s.v[tb][v + 2], s.v[tb][v + 3]};
+            if (quads) {
+                if (p < a.rows) *reinterpret_cast<float4*>(row + p) = make_float4(q[0], q[1], q[2], q[3]);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (p + i < a.rows) row[p + i] = q[i];
+            }
+        }
+    }
+}
+
+template <uint32_t F, int TB, bool FULL, bool CLIP, bool SPLIT = false>
+__global__ __launch_bounds__(64 * kWaves, 2) void gemm_exact(Product a, uint32_t token_tiles, uint32_t row_tiles,
+                                                             uint32_t chunks, float* range_sums, bool quads) {
+    // A group's inputs a stage: [token][half][pair], 16-byte slots swizzled.
+    constexpr uint32_t kStage = 256 * TB;  // float4s
+    __shared__ float4 stages[4 * kStage];
+    const uint32_t lane = threadIdx.x & 63u, half = lane >> 5;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // Uniform, and held so: what follows from them stays in scalar registers.
+    const uint32_t tile_t = __builtin_amdgcn_readfirstlane(blockIdx.x % token_tiles);
+    const uint32_t tile_r = __builtin_amdgcn_readfirstlane((blockIdx.x / token_tiles) % row_tiles);
+    const uint32_t chunk = __builtin_amdgcn_readfirstlane(blockIdx.x / (token_tiles * row_tiles));
+    const uint32_t T = tile_t * 32 * TB, R = (tile_r * kWaves + wave) * kWaveRows;
     const uint32_t G = a.groups;
-    const uint64_t K = static_cast<uint64_t>(G) * 32;
-    const uint32_t r_begin = 32 * chunk / chunks, r_end = 32 * (chunk + 1) / chunks;
-    const uint32_t g_begin = range_lo(r_begin, G), g_end = range_lo(r_end, G);
+    const auto lo_of = [&](uint32_t r) { return (r * G) >> 5; };  // range_lo; G is below 2^24
+    const uint32_t chunk_r = __builtin_amdgcn_readfirstlane(32 * chunk / chunks);
+    const uint32_t g_begin = lo_of(chunk_r);
+    const uint32_t g_end = lo_of(__builtin_amdgcn_readfirstlane(32 * (chunk + 1) / chunks));
     if (g_begin >= g_end) return;  // a chunk of empty ranges (G < 32): nothing to write
+    const uint32_t g_last = g_end - 1;
 
     // Rows and tokens past the product read its last row or token; their
-    // outputs are never stored.
-    const Piece pc = piece_of(a, min(R + lane, a.rows - 1));
+    // outputs are never stored. A wave whose rows all lie past it still
+    // copies its share of the inputs and meets the others.
+    const Piece pc = piece_of(a, min(R + (lane & 31u), a.rows - 1));
     const uint64_t row0 = static_cast<uint64_t>(pc.row) * G;
-    const uint32_t my_token = T + (TT == 64 ? lane : lane & 31u);
-    const float4* xrow = reinterpret_cast<const float4*>(a.x + static_cast<uint64_t>(min(my_token, a.tokens - 1)) * K);
+    // Inputs: of a group's TB x 32 tokens x 8 chunks of 4 ks, thread t copies
+    // chunk c = t % 8 of token t / 8 — eight lanes a token's 128-byte line — its
+    // even ks and its odd ones to their halves of the token's slots. TB = 1
+    // has half as many chunks as threads: the upper 256 take the next group's.
+    const uint32_t ct = (threadIdx.x / 8) % (32 * TB), c = threadIdx.x % 8;
+    constexpr uint32_t kGroupsACopy = TB == 1 ? 2 : 1;  // groups a copy covers
+    const uint32_t copy_group = TB == 1 ? threadIdx.x >> 8 : 0;
+    const float4* const x =
+        reinterpret_cast<const float4*>(a.x) + min(T + ct, a.tokens - 1) * (G * uint64_t{8}) + c;
     float lo = 0.0f, hi = 0.0f;
     if constexpr (CLIP) lo = *a.clip[0], hi = *a.clip[1];
-
-    // Range sums (TT = 64: rows R .. R + 31 and R + 32 .. R + 63 against 64
-    // tokens; TT = 32: s0 alone, rows R .. R + 63 against 32) and totals.
-    constexpr int S = TT == 64 ? 2 : 1;
-    f32x32 s0 = {}, s1 = {};
-    float t[S][32];
+    // A token's eight 16-byte slots: half h's ks 8j + h .. 8j + 6 + h at slot
+    // (4h + j) ^ (token % 8), so a read of one slot for 32 tokens spreads over the banks.
+    float2* const store_at = reinterpret_cast<float2*>(stages + copy_group * kStage + 8 * ct);
+    const uint32_t even_at = 2 * ((c / 2) ^ (ct & 7u)) + (c & 1u), odd_at = 2 * ((4 + c / 2) ^ (ct & 7u)) + (c & 1u);
+    const float4* read_at[4];
 #pragma unroll
-    for (int v = 0; v < 32; ++v)
-#pragma unroll
-        for (int i = 0; i < S; ++i) t[i][v] = 0.0f;
+    for (int j = 0; j < 4; ++j) read_at[j] = stages + 8 * (lane & 31u) + ((4 * half + j) ^ (lane & 7u));
 
-    // The range that ends after group g is the one before `next_r`'s first
-    // group; ranges with no groups (G < 32) hold zero and add nothing.
-    uint32_t next_r = r_begin + 1;
-    while (next_r < r_end && range_lo(next_r, G) <= g_begin) ++next_r;
-
-    // A group's bytes and inputs are loaded a whole group ahead, into one of
-    // two buffers (the loop takes groups in pairs, so each buffer keeps its
-    // registers): at the top of group g every load of group g has been
-    // waited for, and the loads of group g + 1 go out before its products,
-    // so no wait inside them depends on a load issued in the same group.
-    struct Buffer {
-        Raw<F> raw;
-        float4 xq[8];
+    constexpr int kCopies = 2 / kGroupsACopy;  // copies of a pair of groups
+    struct Pair {
+        float4 q[kCopies];
     };
-    auto fetch = [&](Buffer& b, uint32_t g) {
-        b.raw.load(pc.piece, pc.blocks, row0 + g);
+    auto load_x = [&](Pair& p, uint32_t g) {
 #pragma unroll
-        for (int v = 0; v < 8; ++v) b.xq[v] = xrow[8 * g + v];
+        for (int i = 0; i < kCopies; ++i) p.q[i] = x[8 * min(g + i + copy_group, g_last)];
     };
-    bool fresh = true;  // the next product starts a range: its chain from +0
-    auto group = [&](const Buffer& b, uint32_t g) {
-        float w[32], x[32];
-        weights_of(b.raw, w);
+    auto store_x = [&](const Pair& p, uint32_t stage) {
 #pragma unroll
-        for (int v = 0; v < 8; ++v) {
-            float4 q = b.xq[v];
+        for (int i = 0; i < kCopies; ++i) {
+            float4 q = p.q[i];
             if constexpr (CLIP) {
-                q.x = clamp_to(q.x, lo, hi);
-                q.y = clamp_to(q.y, lo, hi);
-                q.z = clamp_to(q.z, lo, hi);
-                q.w = clamp_to(q.w, lo, hi);
+                q.x = clamp_to(q.x, lo, hi), q.y = clamp_to(q.y, lo, hi);
+                q.z = clamp_to(q.z, lo, hi), q.w = clamp_to(q.w, lo, hi);
             }
-            x[4 * v] = q.x;
-            x[4 * v + 1] = q.y;
-            x[4 * v + 2] = q.z;
-            x[4 * v + 3] = q.w;
+            store_at[2 * kStage * (stage + i) + even_at] = make_float2(q.x, q.z);
+            store_at[2 * kStage * (stage + i) + odd_at] = make_float2(q.y, q.w);
         }
-        // A range's first product takes +0 as its accumulator, so the chain
-        // starts from +0 as fma(w, x, +0) does (the sums are never cleared).
-        if (fresh) {
-            const f32x32 zero = {};
-            if constexpr (TT == 64) {
-                s0 = __builtin_amdgcn_mfma_f32_32x32x1f32(w[0], x[0], zero, 1, 0, 0);
-                s1 = __builtin_amdgcn_mfma_f32_32x32x1f32(w[0], x[0], zero, 1, 1, 0);
-            } else {
-                s0 = __builtin_amdgcn_mfma_f32_32x32x1f32(w[0], x[0], zero, 0, 0, 0);
-            }
-        } else {
-            if constexpr (TT == 64) {
-                s0 = __builtin_amdgcn_mfma_f32_32x32x1f32(w[0], x[0], s0, 1, 0, 0);
-                s1 = __builtin_amdgcn_mfma_f32_32x32x1f32(w[0], x[0], s1, 1, 1, 0);
-            } else {
-                s0 = __builtin_amdgcn_mfma_f32_32x32x1f32(w[0], x[0], s0, 0, 0, 0);
-            }
-        }
+    };
+    // Every wave's stores of the next stages before any wave reads them, and
+    // its reads of these before any stores over them.
+    auto meet = [] {
+        __asm__ __volatile__("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        __asm__ __volatile__("" ::: "memory");
+    };
+
+    Sums<TB> s;
+    float t[TB][16];
 #pragma unroll
-        for (int k = 1; k < 32; ++k) {
-            if constexpr (TT == 64) {
-                s0 = __builtin_amdgcn_mfma_f32_32x32x1f32(w[k], x[k], s0, 1, 0, 0);
-                s1 = __builtin_amdgcn_mfma_f32_32x32x1f32(w[k], x[k], s1, 1, 1, 0);
-            } else {
-                s0 = __builtin_amdgcn_mfma_f32_32x32x1f32(w[k], x[k], s0, 0, 0, 0);
+    for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) t[tb][v] = 0.0f;
+    // Range r, the one being summed, and the groups left in it. Below 32
+    // groups a range that holds one holds it alone (group g's is range (32 g +
+    // 31) / G); the empty ones hold zero and add nothing.
+    uint32_t r = chunk_r;
+    if (G < 32) r = __builtin_amdgcn_readfirstlane((32 * g_begin + 31) / G);
+    uint32_t left = G < 32 ? 1u : lo_of(r + 1) - lo_of(r);
+    bool fresh = true;  // the next product starts a range: its chain from +0
+
+    auto group = [&](const HalfRaw<F>& raw, uint32_t stage, uint32_t g) {
+        Half<F> ops;
+        ops.decode(raw, half);
+        const f32x16 zero = {};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            float aw[4];
+            ops.four(j, aw);
+            float4 q[TB];
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb) q[tb] = read_at[j][kStage * stage + 256 * tb];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float bx[TB];
+#pragma unroll
+                for (int tb = 0; tb < TB; ++tb) bx[tb] = i == 0 ? q[tb].x : i == 1 ? q[tb].y : i == 2 ? q[tb].z : q[tb].w;
+                if (j == 0 && i == 0) {
+                    // a range's first product takes +0 as its accumulator, as
+                    // fma(w, x, +0) does (the sums are never cleared)
+                    if (fresh) {
+#pragma unroll
+                        for (int tb = 0; tb < TB; ++tb)
+                            s.v[tb] = __builtin_amdgcn_mfma_f32_32x32x2f32(aw[0], bx[tb], zero, 0, 0, 0);
+                        continue;
+                    }
+                }
+#pragma unroll
+                for (int tb = 0; tb < TB; ++tb)
+                    s.v[tb] = __builtin_amdgcn_mfma_f32_32x32x2f32(aw[i], bx[tb], s.v[tb], 0, 0, 0);
             }
         }
-        fresh = g + 1 == range_lo(next_r, G);
-        if (fresh) {  // range next_r - 1 ends
+        fresh = --left == 0;
+        if (fresh) {  // range r ends
             if constexpr (SPLIT) {
-#pragma unroll
-                for (int v = 0; v < 32; v += 4) {
-                    const uint32_t in_block = 8 * ((v & 15) / 4) + 4 * (lane >> 5);  // rows in_block .. + 3
-                    uint32_t token, p;
-                    if constexpr (TT == 64) {
-                        token = T + 32 * (v / 16) + (lane & 31u), p = R + in_block;
-                    } else {
-                        token = T + (lane & 31u), p = R + 32 * (v / 16) + in_block;
-                    }
-                    if (token >= a.tokens) continue;
-                    float* at = range_sums + (static_cast<uint64_t>(next_r - 1) * a.tokens + token) * a.rows + p;
-                    float q0[4] = {s0[v], s0[v + 1], s0[v + 2], s0[v + 3]};
-                    if (quads) {
-                        if (p < a.rows) *reinterpret_cast<float4*>(at) = make_float4(q0[0], q0[1], q0[2], q0[3]);
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            if (p + i < a.rows) at[i] = q0[i];
-                    }
-                    if constexpr (S == 2) {
-                        float q1[4] = {s1[v], s1[v + 1], s1[v + 2], s1[v + 3]};
-                        if (quads) {
-                            if (p + 32 < a.rows)
-                                *reinterpret_cast<float4*>(at + 32) = make_float4(q1[0], q1[1], q1[2], q1[3]);
-                        } else {
-#pragma unroll
-                            for (int i = 0; i < 4; ++i)
-                                if (p + 32 + i < a.rows) at[32 + i] = q1[i];
-                        }
-                    }
-                }
+                store_sums(a, s, r, R, T, range_sums, quads);
             } else {
 #pragma unroll
-                for (int v = 0; v < 32; ++v) {
-                    const float a0 = s0[v];
-                    t[0][v] = t[0][v] + a0;
-                    if constexpr (S == 2) {
-                        const float a1 = s1[v];
-                        t[S - 1][v] = t[S - 1][v] + a1;
+                for (int tb = 0; tb < TB; ++tb)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) {
+                        const float e = s.v[tb][v];
+                        t[tb][v] = t[tb][v] + e;
                     }
-                }
             }
-            while (next_r < r_end && range_lo(next_r, G) <= g + 1) ++next_r;
+            if (G < 32) {
+                if constexpr (SPLIT) r = __builtin_amdgcn_readfirstlane((32 * (g + 1) + 31) / G);
+                left = 1;
+            } else {
+                ++r;
+                left = lo_of(r + 1) - lo_of(r);
+            }
         }
     };
 
+    // Groups go in pairs: a group's codes are loaded one ahead, into one of
+    // two buffers, a pair's inputs two pairs ahead, into registers, then LDS.
     // Every fetch is issued on every path (past the last group it reads the
     // last group again, unused), so the count of loads in flight at each wait
-    // is the same on every path: a wait for one buffer never waits for the
-    // other's loads.
-    Buffer A, B;
+    // is the same on every path.
+    HalfRaw<F> A, B;
+    Pair px;
+    auto fetch = [&](HalfRaw<F>& b, uint32_t g) { b.load_half(pc.piece, pc.blocks, row0 + min(g, g_last), half); };
+    load_x(px, g_begin);
     fetch(A, g_begin);
-    for (uint32_t g = g_begin; g < g_end; g += 2) {
-        fetch(B, min(g + 1, g_end - 1));
-        group(A, g);
-        if (g + 1 >= g_end) break;
-        fetch(A, min(g + 2, g_end - 1));
-        group(B, g + 1);
+    store_x(px, 0);
+    load_x(px, g_begin + 2);
+    meet();
+    // A pair out of stages `stage`, stage + 1; false after the last group.
+    auto pair = [&](uint32_t stage, uint32_t g) {
+        fetch(B, g + 1);
+        store_x(px, stage ^ 2);
+        load_x(px, g + 4);
+        group(A, stage, g);
+        if (g + 1 >= g_end) return false;
+        fetch(A, g + 2);
+        group(B, stage + 1, g + 1);
+        meet();
+        return g + 2 < g_end;
+    };
+    for (uint32_t g = g_begin; pair(0, g) && pair(2, g + 2); g += 4) {
     }
     if constexpr (SPLIT) return;
 
 #pragma unroll
-    for (int v = 0; v < 32; ++v) {
-        const uint32_t in_block = 8 * ((v & 15) / 4) + 4 * (lane >> 5) + (v & 3);
-        if constexpr (TT == 64) {
-            const uint32_t token = T + 32 * (v / 16) + (lane & 31u), p = R + in_block;
-            if (token < a.tokens) {
-                if (p < a.rows) emit<FULL>(a, p, token, token, t[0][v], (v & 1) ? 0.0f : t[0][v ^ 1]);
-                if (p + 32 < a.rows) emit<FULL>(a, p + 32, token, token, t[S - 1][v], (v & 1) ? 0.0f : t[S - 1][v ^ 1]);
-            }
-        } else {
-            const uint32_t token = T + (lane & 31u), p = R + 32 * (v / 16) + in_block;
-            if (token < a.tokens && p < a.rows) emit<FULL>(a, p, token, token, t[0][v], (v & 1) ? 0.0f : t[0][v ^ 1]);
-        }
+    for (int tb = 0; tb < TB; ++tb) {
+        const uint32_t token = T + 32 * tb + (lane & 31u);
+        if (token < a.tokens) emit_block<FULL>(a, R, token, t[tb]);
     }
 }
 
@@ -645,46 +873,43 @@ void go_exact_short(const Product& a, const Plan& plan, hipStream_t stream) {
         hipLaunchKernelGGL((gemm_exact_short<F, true, true>), grid, block, 0, stream, a, tt);
 }
 
-template <uint32_t F, uint32_t TT>
+template <uint32_t F, int TB>
 void go_exact_tile(const Product& a, const Plan& plan, float* range_sums, hipStream_t stream) {
     const dim3 grid(static_cast<uint32_t>(plan.workgroups)), block(64 * kWaves);
     const uint32_t tt = plan.token_tiles, rt = plan.row_tiles, ch = plan.chunks;
     if (range_sums) {  // a split product has no options and is not gated
         const bool quads = a.rows % 4 == 0 && reinterpret_cast<uintptr_t>(range_sums) % 16 == 0;
-        hipLaunchKernelGGL((gemm_exact<F, TT, false, false, true>), grid, block, 0, stream, a, tt, rt, ch, range_sums,
+        hipLaunchKernelGGL((gemm_exact<F, TB, false, false, true>), grid, block, 0, stream, a, tt, rt, ch, range_sums,
                            quads);
     } else if (plain_epilogue(a)) {
-        hipLaunchKernelGGL((gemm_exact<F, TT, false, false>), grid, block, 0, stream, a, tt, rt, 1u, nullptr, false);
+        hipLaunchKernelGGL((gemm_exact<F, TB, false, false>), grid, block, 0, stream, a, tt, rt, 1u, nullptr, false);
     } else if (!clipped(a)) {
-        hipLaunchKernelGGL((gemm_exact<F, TT, true, false>), grid, block, 0, stream, a, tt, rt, 1u, nullptr, false);
+        hipLaunchKernelGGL((gemm_exact<F, TB, true, false>), grid, block, 0, stream, a, tt, rt, 1u, nullptr, false);
     } else {
-        hipLaunchKernelGGL((gemm_exact<F, TT, true, true>), grid, block, 0, stream, a, tt, rt, 1u, nullptr, false);
+        hipLaunchKernelGGL((gemm_exact<F, TB, true, true>), grid, block, 0, stream, a, tt, rt, 1u, nullptr, false);
     }
 }
 
 template <uint32_t F>
 void go_exact(const Product& a, const Plan& plan, float* range_sums, hipStream_t stream) {
     if constexpr (F != kF32) {
-        if (plan.tile_tokens == 64) return go_exact_tile<F, 64>(a, plan, range_sums, stream);
+        if (plan.tile_tokens == 64) return go_exact_tile<F, 2>(a, plan, range_sums, stream);
     }
-    go_exact_tile<F, 32>(a, plan, range_sums, stream);
+    go_exact_tile<F, 1>(a, plan, range_sums, stream);
 }
 
 }  // namespace
 
-// Tiles of 256 rows (four waves of 64) by 64 or 32 tokens, token tile first,
-// so the tiles reading one row tile's weights run together. A wave's time is
-// its walk through K, and a SIMD's waves share its matrix core, so a step
-// takes as many rounds as its most loaded SIMD holds waves: 64 x 64 waves
-// where they give no more rounds than 64 x 32 waves give half-length ones
-// (one wave of 64 x 64 a SIMD, two chains of products, measured faster than
-// two of 64 x 32, one chain each: C4 98.6 against 93.4 TFLOP/s), else 64 x
-// 32 — Llama 3.2 1B's QKV at 2,048 tokens: 1,536 waves of 64 x 64 on 1,024
-// SIMDs are two rounds, 3,072 of 64 x 32 one and a half. F32 always by 32 (its
-// 32 dwords a group beside 64 tokens' sums would not fit two waves' registers).
+// Tiles of 256 rows (eight waves of 32) by 64 or 32 tokens, token tile first,
+// so the tiles reading one row tile's weights run together. A SIMD's waves
+// share its matrix core, so a step takes as many rounds as its most loaded
+// SIMD holds pairs of waves: 64 tokens where they give no more rounds than 32
+// give half-length ones (a decoded weight then serves twice the products),
+// else 32 — Llama 3.2 1B's QKV at 2,048 tokens: 1,536 pairs by 64 on 1,024
+// SIMDs are two rounds, 3,072 by 32 one and a half. F32 always by 32.
 void plan_gemm_exact(const Product& a, uint32_t format, uint32_t compute_units, bool split, Plan* plan) {
     *plan = Plan{};
-    const uint64_t wave_rows = (a.rows + kWaveRows - 1) / kWaveRows;
+    const uint64_t wave_rows = (a.rows + 63) / 64;
     const uint64_t simds = 4ull * compute_units;
     const uint64_t rounds64 = (wave_rows * ((a.tokens + 63) / 64) + simds - 1) / simds;
     const uint64_t rounds32 = (wave_rows * ((a.tokens + 31) / 32) + simds - 1) / simds;  // half-length rounds

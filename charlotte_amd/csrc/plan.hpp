@@ -28,7 +28,7 @@ enum Kernel : uint32_t {
     kGemmSplit = 17,    // prefill split along K, then the ordered combine
     kGemmMfma = 18,     // prefill on the matrix cores, x split into two f16 parts
     kGemmShort = 19,    // prefill of a short step: 16 or 8 rows x 32 tokens, K split among the waves
-    kGemmExact = 20,    // prefill on the matrix cores' K = 1 f32 instruction, the canonical order
+    kGemmExact = 20,    // prefill on the matrix cores' f32 instructions, the canonical order
     kGemmExactSplit = 21,  // the same split along K, then the ordered combine
     kGemmExactShort = 22,  // a short step on the matrix cores: 32 x 32, K split among 8 waves
 };

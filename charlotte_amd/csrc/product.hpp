@@ -168,6 +168,29 @@ __device__ __forceinline__ void put(float v, float* at) {
         *at = v;
 }
 
+// The value of a gated output from its gate and up totals.
+__device__ __forceinline__ float gated_value(const Product& a, float g, float u) {
+    if (clipped(a)) {
+        const float lo = *a.clip[2], hi = *a.clip[3];
+        g = clamp_to(g, lo, hi), u = clamp_to(u, lo, hi);
+    }
+    return activate(a.activation, g) * u;
+}
+
+// The value of any other epilogue's output, index o in its token's row.
+__device__ __forceinline__ float finished_value(const Product& a, uint32_t o, uint32_t in_token, float total) {
+    float y = total;
+    if (a.epilogue == kGatedByInput) {
+        y = activate(a.activation, y) *
+            a.gate_input[static_cast<uint64_t>(in_token) * a.gate_stride + a.gate_column + o];
+    } else if (a.epilogue == kWrite) {
+        if (clipped(a)) y = clamp_to(y, *a.clip[2], *a.clip[3]);
+        if (a.bias) y = y + a.bias[o];
+        if (a.activated) y = activate(a.activation, y);
+    }
+    return y;
+}
+
 template <bool FULL, bool THROUGH = false>
 __device__ __forceinline__ void emit(const Product& a, uint32_t p, uint32_t token, uint32_t in_token, float total,
                                      float partner) {
@@ -177,25 +200,61 @@ __device__ __forceinline__ void emit(const Product& a, uint32_t p, uint32_t toke
     }
     if (a.epilogue == kGated) {
         if (p & 1u) return;
-        float g = total, u = partner;
-        if (clipped(a)) {
-            const float lo = *a.clip[2], hi = *a.clip[3];
-            g = clamp_to(g, lo, hi), u = clamp_to(u, lo, hi);
-        }
-        put<THROUGH>(activate(a.activation, g) * u, &a.m[0].out[static_cast<uint64_t>(token) * a.m[0].out_width + (p >> 1)]);
+        put<THROUGH>(gated_value(a, total, partner),
+                     &a.m[0].out[static_cast<uint64_t>(token) * a.m[0].out_width + (p >> 1)]);
         return;
     }
     const Place w = place_of(a, p, token);
-    float y = total;
-    if (a.epilogue == kGatedByInput) {
-        y = activate(a.activation, y) *
-            a.gate_input[static_cast<uint64_t>(in_token) * a.gate_stride + a.gate_column + w.o];
-    } else if (a.epilogue == kWrite) {
-        if (clipped(a)) y = clamp_to(y, *a.clip[2], *a.clip[3]);
-        if (a.bias) y = y + a.bias[w.o];
-        if (a.activated) y = activate(a.activation, y);
+    put<THROUGH>(finished_value(a, w.o, in_token, total), w.at);
+}
+
+// A lane's sixteen rows of a 32-row block from R (R a multiple of 32, the
+// same for the whole wave) of one token, as the 32 x 32 matrix instructions
+// leave them: register v is row R + 8 (v / 4) + 4 (lane / 32) + v % 4. Where
+// the block lies in one member whole and its places are so aligned, four rows
+// go out as one 16-byte store (gated: two outputs as one of 8): a store's
+// lanes are tokens, each its own line, so a quarter of the stores is a
+// quarter of the lines touched. Else a row at a time.
+template <bool FULL>
+__device__ __forceinline__ void emit_block(const Product& a, uint32_t R, uint32_t token, const float (&t)[16]) {
+    const uint32_t p = R + 4 * ((threadIdx.x & 63u) >> 5);
+    const bool whole = R + 32 <= a.rows && (a.members < 2 || R + 32 <= a.m[1].first || R >= a.m[1].first) &&
+                       (a.members < 3 || R + 32 <= a.m[2].first || R >= a.m[2].first);
+    if (FULL && a.epilogue == kGated) {
+        float* const at = &a.m[0].out[static_cast<uint64_t>(token) * a.m[0].out_width + (p >> 1)];
+        const bool aligned = R + 32 <= a.rows && reinterpret_cast<uintptr_t>(a.m[0].out) % 8 == 0 && a.m[0].out_width % 2 == 0;
+#pragma unroll
+        for (int v = 0; v < 16; v += 4) {
+            const float y0 = gated_value(a, t[v], t[v + 1]), y1 = gated_value(a, t[v + 2], t[v + 3]);
+            if (aligned) {
+                *reinterpret_cast<float2*>(at + v) = make_float2(y0, y1);
+            } else {
+                if (p + 2 * v < a.rows) at[v] = y0;
+                if (p + 2 * v + 2 < a.rows) at[v + 1] = y1;
+            }
+        }
+        return;
     }
-    put<THROUGH>(y, w.at);
+    const Place first = place_of(a, min(R, a.rows - 1), token);  // R's: its member is the block's where `whole`
+    if (whole && reinterpret_cast<uintptr_t>(first.at) % 16 == 0) {
+        float* const at = first.at + (p - R);
+        const uint32_t o = first.o + (p - R);
+#pragma unroll
+        for (int v = 0; v < 16; v += 4) {
+            float y[4] = {t[v], t[v + 1], t[v + 2], t[v + 3]};
+            if constexpr (FULL) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) y[i] = finished_value(a, o + 2 * v + i, token, y[i]);
+            }
+            *reinterpret_cast<float4*>(at + 2 * v) = make_float4(y[0], y[1], y[2], y[3]);
+        }
+        return;
+    }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        const uint32_t row = p + 8 * (v / 4) + v % 4;
+        if (row < a.rows) emit<FULL>(a, row, token, token, t[v], 0.0f);
+    }
 }
 
 }  // namespace chm

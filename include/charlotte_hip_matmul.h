@@ -118,10 +118,10 @@ typedef enum {
  * order above (split along K where the gate and the caller's range sums
  * allow), bit-exact and batch-invariant: a drop-in caller keeps the
  * reference's decode = prefill guarantee whatever workspace it sets. For a
- * step that does not split, AUTO takes the matrix cores' K = 1 f32
- * instruction (GEMM_EXACT: each range's chain one fused multiply-add a k, as
- * the VALU tile adds it, on 64-row waves) where the step gives it at least
- * three waves a compute unit; else the same chains split among a workgroup's
+ * step that does not split, AUTO takes the matrix cores' f32
+ * instructions (GEMM_EXACT: each range's chain one fused multiply-add a k, as
+ * the VALU tile adds it, in 256-row tiles) where the step gives it at least
+ * three 64-row, 64- or 32-token shares a compute unit; else the same chains split among a workgroup's
  * waves (GEMM_EXACT_SHORT: 32 rows by 32 tokens, or 16 by 16 where the larger
  * tiles would leave compute units idle, eight waves of four ranges, the range
  * sums combined in LDS). A step that splits runs its chunks of
