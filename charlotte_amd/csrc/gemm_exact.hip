@@ -52,76 +52,11 @@ namespace chm {
 
 namespace {
 
-typedef float f32x32 __attribute__((ext_vector_type(32)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kWaveRows = 32;   // rows a wave
 constexpr uint32_t kWaves = 8;       // waves a workgroup, each its own 32 rows
-
-// Four weights from four code bytes as the decodes' chain4 makes them: two
-// codes a v_perm_b32 as binary16 1024 + b, then one v_fma_mix_f32 a weight,
-// fma(1024 + b, scale, offset) — one rounding of a value f32 holds exactly.
-__device__ __forceinline__ void weights4(uint32_t codes, float scale, float offset, float* w) {
-    const half2_t a = lift(codes, kLowPair), b = lift(codes, kHighPair);
-    w[0] = __builtin_fmaf(static_cast<float>(a.x), scale, offset);
-    w[1] = __builtin_fmaf(static_cast<float>(a.y), scale, offset);
-    w[2] = __builtin_fmaf(static_cast<float>(b.x), scale, offset);
-    w[3] = __builtin_fmaf(static_cast<float>(b.y), scale, offset);
-}
-
-// The 32 exact weights of a group as loaded: the values of formats.hpp's
-// weight(), which the VALU tile stages. Q4_0, Q8_0 and Q6_K by the lift of
-// decode.hpp's chain_q4_0, chain_q8_0 and chain_q6_k (1.75 instructions a
-// weight against weight()'s 3), the others by weight(). The short-step tiles'.
-template <uint32_t F>
-__device__ __forceinline__ void weights_of(const Raw<F>& r, float* w) {
-    if constexpr (F == kQ4_0) {
-        // (1024 + q) d - 1032 d; high nibbles as bytes 16 q: (1024 + 16 q) (d / 16) - 72 d
-        const float d = half_to_float(r.d);
-        const float low_offset = -1032.0f * d, d16 = d * 0.0625f, high_offset = -72.0f * d;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            weights4(r.w[c] & 0x0F0F0F0Fu, d, low_offset, w + 4 * c);
-            weights4(r.w[c] & 0xF0F0F0F0u, d16, high_offset, w + 16 + 4 * c);
-        }
-    } else if constexpr (F == kQ4_1) {
-        const Q4_1Group g = group_of(Q4_1Bytes{make_uint4(r.w[0], r.w[1], r.w[2], r.w[3]), r.dm});
-#pragma unroll
-        for (int l = 0; l < 32; ++l) w[l] = weight(g, l);
-    } else if constexpr (F == kQ8_0) {
-        // q + 128 (the sign bit flipped) lifted: fma(1152 + q, d, -1152 d) = q d
-        const float d = half_to_float(r.d), offset = -1152.0f * d;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) weights4(r.w[c] ^ 0x80808080u, d, offset, w + 4 * c);
-    } else if constexpr (F == kQ6_K) {
-        // the 6-bit codes assembled as chain_q6_k assembles them, then
-        // fma(1024 + q, scale, -1056 scale) = (q - 32) scale
-        const float d = half_to_float(r.d);
-        const float first = d * static_cast<float>(static_cast<int8_t>(r.sc & 0xFFu));
-        const float second = d * static_cast<float>(static_cast<int8_t>((r.sc >> 8) & 0xFFu));
-        const float first_offset = -1056.0f * first, second_offset = -1056.0f * second;
-        const uint32_t a0 = r.hi[0] & 0x33333333u, a1 = r.hi[1] & 0x33333333u;
-        const uint32_t b0 = (r.hi[0] >> 2) & 0x33333333u, b1 = (r.hi[1] >> 2) & 0x33333333u;
-        constexpr uint32_t kNib = 0x0F0F0F0Fu;
-        weights4(bitfield_insert(kNib, r.lo[0], a0 << 4), first, first_offset, w + 0);
-        weights4(bitfield_insert(kNib, r.lo[1], a1 << 4), first, first_offset, w + 4);
-        weights4(bitfield_insert(kNib, r.lo[2], b0 << 4), first, first_offset, w + 8);
-        weights4(bitfield_insert(kNib, r.lo[3], b1 << 4), first, first_offset, w + 12);
-        weights4(bitfield_insert(kNib, r.lo[0] >> 4, a0), second, second_offset, w + 16);
-        weights4(bitfield_insert(kNib, r.lo[1] >> 4, a1), second, second_offset, w + 20);
-        weights4(bitfield_insert(kNib, r.lo[2] >> 4, b0), second, second_offset, w + 24);
-        weights4(bitfield_insert(kNib, r.lo[3] >> 4, b1), second, second_offset, w + 28);
-    } else if constexpr (F == kF32) {
-#pragma unroll
-        for (int l = 0; l < 32; ++l) w[l] = __uint_as_float(r.w[l]);
-    } else {
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            w[2 * i] = F == kF16 ? half_to_float(r.w[i] & 0xFFFFu) : bf16_low(r.w[i]);
-            w[2 * i + 1] = F == kF16 ? half_to_float(r.w[i] >> 16) : bf16_high(r.w[i]);
-        }
-    }
-}
 
 // The upper half-wave of `a` against the lower of `b`: afterwards a holds the
 // two lower halves (a's, then b's), b the two upper ones.
@@ -522,329 +457,496 @@ __global__ __launch_bounds__(64 * kWaves, 2) void gemm_exact(Product a, uint32_t
 }
 
 
+// A lane's share of one row's group for the K = 4 instruction: lane quarter q
+// (lanes 16 q .. 16 q + 15) takes ks q, 4 + q, ..., 28 + q, its eight weights
+// weight()'s values: eight(q, w) makes them from the group's bytes, byte q of
+// each code dword, two dwords at a time.
+template <uint32_t F>
+struct Quarter;
+
+// Byte q of `first` and of `second` as the low bytes of a dword's halves.
+__device__ __forceinline__ uint32_t bytes_of(uint32_t first, uint32_t second, uint32_t q) {
+    return __builtin_amdgcn_perm(second, first, 0x0C040C00u + 0x00010001u * q);
+}
+
+template <>
+struct Quarter<kQ4_0> : Raw<kQ4_0> {
+    __device__ __forceinline__ void eight(uint32_t q, float* o) const {
+        const float s = half_to_float(d), s16 = 16.0f * s, low = -1032.0f * s, high = -72.0f * s;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t p = bytes_of(w[2 * i], w[2 * i + 1], q);
+            // (64 + l / 16) 16 d - 1032 d and (64 + h) d - 72 d, as Half<kQ4_0>
+            const half2_t l = __builtin_bit_cast(half2_t, and_or(p, 0x000F000Fu, 0x54005400u));
+            const half2_t h = __builtin_bit_cast(half2_t, and_or(p, 0x00F000F0u, 0x54005400u));
+            o[2 * i] = __builtin_fmaf(static_cast<float>(l.x), s16, low);
+            o[2 * i + 1] = __builtin_fmaf(static_cast<float>(l.y), s16, low);
+            o[4 + 2 * i] = __builtin_fmaf(static_cast<float>(h.x), s, high);
+            o[5 + 2 * i] = __builtin_fmaf(static_cast<float>(h.y), s, high);
+        }
+    }
+};
+
+template <>
+struct Quarter<kQ4_1> : Raw<kQ4_1> {
+    __device__ __forceinline__ void eight(uint32_t q, float* o) const {
+        const float s = half_to_float(dm & 0xFFFFu), m = half_to_float(dm >> 16), s16 = s * 0.0625f;
+        const half2_t base = {1024.0f16, 1024.0f16};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t p = bytes_of(w[2 * i], w[2 * i + 1], q);
+            const half2_t l = __builtin_bit_cast(half2_t, and_or(p, 0x000F000Fu, 0x64006400u)) - base;
+            const half2_t h = __builtin_bit_cast(half2_t, and_or(p, 0x00F000F0u, 0x64006400u)) - base;
+            o[2 * i] = __builtin_fmaf(static_cast<float>(l.x), s, m);
+            o[2 * i + 1] = __builtin_fmaf(static_cast<float>(l.y), s, m);
+            o[4 + 2 * i] = __builtin_fmaf(static_cast<float>(h.x), s16, m);
+            o[5 + 2 * i] = __builtin_fmaf(static_cast<float>(h.y), s16, m);
+        }
+    }
+};
+
+template <>
+struct Quarter<kQ8_0> : Raw<kQ8_0> {
+    __device__ __forceinline__ void eight(uint32_t q, float* o) const {
+        const float s = half_to_float(d), offset = -1152.0f * s;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            // q + 128 (the sign bit flipped) under 0x64: 1152 + q
+            const half2_t u = __builtin_bit_cast(half2_t, bytes_of(w[2 * i], w[2 * i + 1], q) ^ 0x64806480u);
+            o[2 * i] = __builtin_fmaf(static_cast<float>(u.x), s, offset);
+            o[2 * i + 1] = __builtin_fmaf(static_cast<float>(u.y), s, offset);
+        }
+    }
+};
+
+template <>
+struct Quarter<kQ6_K> : Raw<kQ6_K> {
+    __device__ __forceinline__ void eight(uint32_t q, float* o) const {
+        const float s = half_to_float(d);
+        const float first = s * static_cast<float>(static_cast<int8_t>(sc & 0xFFu));
+        const float second = s * static_cast<float>(static_cast<int8_t>((sc >> 8) & 0xFFu));
+        const float first_offset = -1056.0f * first, second_offset = -1056.0f * second;
+        // the pairs' byte m = 4 (c % 2) + q holds dword c's: bits 0, 2 for the
+        // low nibbles of dwords 0-1 and 2-3, bits 4, 6 for their high ones
+        const uint32_t p01 = bytes_of(lo[0], lo[1], q), p23 = bytes_of(lo[2], lo[3], q), ph = bytes_of(hi[0], hi[1], q);
+        constexpr uint32_t kNib = 0x000F000Fu;
+        const uint32_t codes[4] = {bitfield_insert(kNib, p01, ph << 4), bitfield_insert(kNib, p23, ph << 2),
+                                   bitfield_insert(kNib, p01 >> 4, ph), bitfield_insert(kNib, p23 >> 4, ph >> 2)};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const half2_t u = __builtin_bit_cast(half2_t, and_or(codes[i], 0x003F003Fu, 0x64006400u));
+            const float scale = i < 2 ? first : second, offset = i < 2 ? first_offset : second_offset;
+            o[2 * i] = __builtin_fmaf(static_cast<float>(u.x), scale, offset);
+            o[2 * i + 1] = __builtin_fmaf(static_cast<float>(u.y), scale, offset);
+        }
+    }
+};
+
+template <>
+struct Quarter<kF32> {  // the quarter's own eight values
+    uint32_t w[8];
+    __device__ __forceinline__ void eight(uint32_t, float* o) const {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) o[j] = __uint_as_float(w[j]);
+    }
+};
+
+// F16 and BF16: value q of each four, half q % 2 of dword q / 2 of two.
+template <uint32_t F>
+struct QuarterHalves : Raw<F> {
+    __device__ __forceinline__ void eight(uint32_t q, float* o) const {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t first = this->w[2 * j], second = this->w[2 * j + 1];
+            if constexpr (F == kF16)
+                o[j] = half_to_float(__builtin_amdgcn_perm(second, first, 0x0C0C0100u + 0x0202u * q));
+            else
+                o[j] = __uint_as_float(__builtin_amdgcn_perm(second, first, 0x01000C0Cu + 0x02020000u * q));
+        }
+    }
+};
+template <>
+struct Quarter<kF16> : QuarterHalves<kF16> {};
+template <>
+struct Quarter<kBF16> : QuarterHalves<kBF16> {};
+
+// How sixteen rows' codes reach a wave, kBatch groups at a time: loaded by
+// lanes that read a row's bytes side by side (the four lanes that decode a
+// row's group would read the same bytes four times, sixteen lines a quarter
+// of the wave), stored in the wave's LDS stage, and read back by each lane a
+// group at a time. The quantized formats: four groups, lane l row l / 4's group
+// l % 4; a record's 16-byte words at place 4 row + (group ^ (row / 2 % 4)),
+// so that a read of one group for sixteen rows spreads over the banks.
+template <uint32_t F>
+struct Codes {
+    static constexpr int kBatch = 4;
+    static constexpr uint32_t kWide = F == kQ8_0 ? 2 : 1;                                 // 16-byte words a record
+    static constexpr uint32_t kWords = 64 * (4 * kWide + (F == kQ6_K ? 2 : 0) + 1);  // LDS words
+    Raw<F> raw;
+    static __device__ __forceinline__ uint32_t load_row(uint32_t lane) { return lane >> 2; }
+    __device__ __forceinline__ void load(const uint8_t* piece, uint64_t blocks, uint64_t row0, uint32_t g, uint32_t last,
+                                         uint32_t lane) {
+        raw.load(piece, blocks, row0 + min(g + (lane & 3u), last));
+    }
+    __device__ __forceinline__ void put(float* stage, uint32_t lane) const {
+        uint4* const wide = reinterpret_cast<uint4*>(stage);
+        const uint32_t row = lane >> 2, at = 4 * row + ((lane ^ (row >> 1)) & 3u);
+        uint32_t tail;
+        if constexpr (F == kQ6_K) {
+            wide[at] = make_uint4(raw.lo[0], raw.lo[1], raw.lo[2], raw.lo[3]);
+            reinterpret_cast<uint2*>(stage + 256)[lane] = make_uint2(raw.hi[0], raw.hi[1]);
+            tail = raw.sc | (raw.d << 16);
+        } else {
+#pragma unroll
+            for (uint32_t i = 0; i < kWide; ++i)
+                wide[64 * i + at] = make_uint4(raw.w[4 * i], raw.w[4 * i + 1], raw.w[4 * i + 2], raw.w[4 * i + 3]);
+            if constexpr (F == kQ4_1)
+                tail = raw.dm;
+            else
+                tail = raw.d;
+        }
+        reinterpret_cast<uint32_t*>(stage + kWords - 64)[lane] = tail;
+    }
+    static __device__ __forceinline__ void get(Quarter<F>& out, const float* stage, uint32_t j, uint32_t lane) {
+        const uint4* const wide = reinterpret_cast<const uint4*>(stage);
+        const uint32_t row = lane & 15u, at = 4 * row + (j ^ ((row >> 1) & 3u));
+        const uint32_t tail = reinterpret_cast<const uint32_t*>(stage + kWords - 64)[4 * row + j];
+        if constexpr (F == kQ6_K) {
+            const uint4 l = wide[at];
+            const uint2 h = reinterpret_cast<const uint2*>(stage + 256)[4 * row + j];
+            out.lo[0] = l.x, out.lo[1] = l.y, out.lo[2] = l.z, out.lo[3] = l.w;
+            out.hi[0] = h.x, out.hi[1] = h.y;
+            out.sc = tail & 0xFFFFu, out.d = tail >> 16;
+        } else {
+#pragma unroll
+            for (uint32_t i = 0; i < kWide; ++i) {
+                const uint4 c = wide[64 * i + at];
+                out.w[4 * i] = c.x, out.w[4 * i + 1] = c.y, out.w[4 * i + 2] = c.z, out.w[4 * i + 3] = c.w;
+            }
+            if constexpr (F == kQ4_1)
+                out.dm = tail;
+            else
+                out.d = tail;
+        }
+    }
+};
+
+// F16 and BF16: a group, 64 bytes a row, lane l row l / 4's 16 bytes l % 4.
+template <uint32_t F>
+struct HalfCodes {
+    static constexpr int kBatch = 1;
+    static constexpr uint32_t kWords = 256;
+    uint32_t raw[4];
+    static __device__ __forceinline__ uint32_t load_row(uint32_t lane) { return lane >> 2; }
+    __device__ __forceinline__ void load(const uint8_t* piece, uint64_t, uint64_t row0, uint32_t g, uint32_t last,
+                                         uint32_t lane) {
+        const uint4 c = reinterpret_cast<const uint4*>(piece + 64 * (row0 + min(g, last)))[lane & 3u];
+        raw[0] = c.x, raw[1] = c.y, raw[2] = c.z, raw[3] = c.w;
+    }
+    __device__ __forceinline__ void put(float* stage, uint32_t lane) const {
+        reinterpret_cast<uint4*>(stage)[(lane & ~3u) + ((lane ^ (lane >> 3)) & 3u)] =
+            make_uint4(raw[0], raw[1], raw[2], raw[3]);
+    }
+    static __device__ __forceinline__ void get(Quarter<F>& out, const float* stage, uint32_t, uint32_t lane) {
+        const uint4* const wide = reinterpret_cast<const uint4*>(stage);
+        const uint32_t row = lane & 15u;
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            const uint4 c = wide[4 * row + (i ^ ((row >> 1) & 3u))];
+            out.w[4 * i] = c.x, out.w[4 * i + 1] = c.y, out.w[4 * i + 2] = c.z, out.w[4 * i + 3] = c.w;
+        }
+    }
+};
+template <>
+struct Codes<kF16> : HalfCodes<kF16> {};
+template <>
+struct Codes<kBF16> : HalfCodes<kBF16> {};
+
+// Where element e of a 32-value line's chunk c (values 4c .. 4c + 3, e = k % 4)
+// goes in operand order, and where a lane of quarter q reads values q, 4 + q,
+// ..: [line][q][j], 16-byte slot 2q + j / 4 of a line's eight at (2q + j / 4) ^
+// (line % 8), so that a read of one slot for 16 lines spreads over the banks.
+__device__ __forceinline__ uint32_t operand_word(uint32_t line, uint32_t c, uint32_t e) {
+    return 32 * line + 4 * ((2 * e + (c >> 2)) ^ (line & 7u)) + (c & 3u);
+}
+__device__ __forceinline__ uint32_t operand_slot(uint32_t line, uint32_t q, uint32_t i) {
+    return 8 * line + ((2 * q + i) ^ (line & 7u));
+}
+
+// F32: a group, 128 bytes a row, in operand order as the inputs are.
+template <>
+struct Codes<kF32> {
+    static constexpr int kBatch = 1;
+    static constexpr uint32_t kWords = 512;
+    float4 raw[2];
+    static __device__ __forceinline__ uint32_t load_row(uint32_t lane) { return lane >> 3; }  // and 8 past it
+    __device__ __forceinline__ void load(const uint8_t* const (&piece)[2], const uint64_t (&row0)[2], uint32_t g,
+                                         uint32_t last, uint32_t lane) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            raw[i] = reinterpret_cast<const float4*>(piece[i] + 128 * (row0[i] + min(g, last)))[lane & 7u];
+    }
+    __device__ __forceinline__ void put(float* stage, uint32_t lane) const {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t line = 8 * i + (lane >> 3), c = lane & 7u;
+            stage[operand_word(line, c, 0)] = raw[i].x;
+            stage[operand_word(line, c, 1)] = raw[i].y;
+            stage[operand_word(line, c, 2)] = raw[i].z;
+            stage[operand_word(line, c, 3)] = raw[i].w;
+        }
+    }
+    static __device__ __forceinline__ void get(Quarter<kF32>& out, const float* stage, uint32_t, uint32_t lane) {
+        const uint4* const at = reinterpret_cast<const uint4*>(stage);
+#pragma unroll
+        for (uint32_t i = 0; i < 2; ++i) {
+            const uint4 c = at[operand_slot(lane & 15u, lane >> 4, i)];
+            out.w[4 * i] = c.x, out.w[4 * i + 1] = c.y, out.w[4 * i + 2] = c.z, out.w[4 * i + 3] = c.w;
+        }
+    }
+};
+
 // gemm_exact_short — a short step on the matrix cores: the canonical order
 // with K split among a workgroup's waves, as gemm_short splits it on the
 // VALU. A step of few tokens gives gemm_exact few waves, each walking all of
-// K as one chain of dependent matrix instructions (C6's 2,048 x 8,192 at 32
-// tokens: 32 waves); here a workgroup takes 32 rows x 32 tokens and its
-// eight waves four of the 32 ranges each, as two pairs. A pair's two chains
-// run in one v_mfma_f32_32x32x1_2b_f32 (K = 1, two 32 x 32 blocks, one fused
-// multiply-add an element): block b is range r_begin + 2 p + b, its A (row R
-// + l % 32) and B (token T + l % 32) from lanes 32 b .. 32 b + 31, each lane
-// decoding its own range's group, and register v holds block v / 16's row 8
-// ((v % 16) / 4) + 4 (l / 32) + v % 4, column l % 32. Step j of a pair is
-// group j of both ranges; where one range is a group shorter than the other
-// (the two differ by at most one), its block's lanes take -0 and +0 at the
-// pair's last step: fma(-0, +0, acc) is acc for every acc (acc + -0 = acc).
+// K; here a workgroup takes RB x 16 rows by TB x 16 tokens and its eight
+// waves four of the 32 ranges each. A range's chain runs on
+// v_mfma_f32_16x16x4_f32 (K = 4, four fused multiply-adds an element in k
+// order: harness.hip's mfma_chain_check): lane quarter q supplies ks 4j + q
+// of row R + l % 16 as A (Quarter) and of token T + l % 16 as B, and register
+// v of block (rb, tb) is row 4 (l / 16) + v, column l % 16.
 //
-// A step's inputs (two groups x 32 tokens x 128 bytes) reach the wave's LDS
-// stage by eight copies (global_load_lds, 1 KB each: 8 tokens' whole lines of
-// one group), where loading them into registers took eight loads a group
-// touching 32 lines each; token t's 16-byte chunk c lies at position c ^ (t %
-// 8) of its 128 bytes, so a read of one chunk for 32 tokens spreads over the
-// banks. Two stages a wave: a step's loads are waited for (the compiler's
-// wait, which covers its copies, issued before them) before the next step's
-// go out, in flight under this step's chain. The pairs' sums stay in
-// registers through K; then, after a barrier, the stages' LDS holds the range
-// sums ([range][register][lane]: 128 KB, one workgroup a CU), and after a
-// second each thread adds two registers' 32 range sums in order from zero,
-// skipping empty ones (G < 32) — rows p, p + 1 of one token, so a gated pair's
-// totals meet in the thread: gemm_canonical's order, its bits.
-constexpr uint32_t kShortWaves = 8;  // waves a workgroup, two pairs of ranges each
-constexpr uint32_t kShortTile = 32;  // rows, and tokens, a workgroup
-
-template <uint32_t F, bool FULL, bool CLIP>
-__global__ __launch_bounds__(64 * kShortWaves, 1) void gemm_exact_short(Product a, uint32_t token_tiles) {
-    __shared__ float4 lds[32 * 16 * 64 / 4];  // the stages (16 KB a wave), then the range sums (128 KB)
-    static_assert(kShortWaves * 2 * 512 == 32 * 16 * 64 / 4, "two stages of 8 KB a wave fill the range sums' LDS");
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, half = lane >> 5;
-    const uint32_t T = (blockIdx.x % token_tiles) * kShortTile, R = (blockIdx.x / token_tiles) * kShortTile;
+// A wave copies what it multiplies itself — its rows' codes (Codes), and a
+// group's inputs, eight lanes a token's 128-byte line — through its own LDS
+// stage, where lanes find them in operand order; loads run four groups
+// ahead. At a range's end its sums go to LDS ([range][block][lane], 16 bytes a
+// lane), the wave's last range's (wave 0: its four ranges' total, added in
+// order from zero) to its stage, no longer needed. After a barrier each
+// thread adds two rows' sums in order, skipping empty ranges (G < 32) — rows
+// p, p + 1 of one token, so a gated pair's totals meet in the thread:
+// gemm_canonical's order, its bits.
+//
+// What bounds it: the f32 products and the VALU take turns on a SIMD
+// (above): 8 products of 32 cycles a 16 x 16 block and group, beside 18 VALU
+// instructions of Q4_0 decode a 16-row group and a few of addresses; then the
+// L1's lines (a row's group read by the four lanes that decode it cost 26
+// against 17 us at 16,384 x 2,048 x 5 tokens) and, at few groups a wave, the
+// launch, the first loads' round trip and the combine. Measured against the
+// K = 1 forms (a pair of ranges, or four, the blocks of one instruction, two
+// groups' inputs staged by LDS copies), us: Q4_0 16,384 x 2,048 at 5 tokens
+// 33.6 -> 16.8, 8,192 x 2,048 at 16 / 64 14.0 -> 11.2 / 34.6 -> 32.2, 2,048 x
+// 8,192 at 5 / 32 19.7 -> 15.9 / 20.5 -> 16.4, 4,096 x 2,048 x 32 13.6 -> 10.5,
+// 2,048 x 2,048 x 32 7.4 -> 7.1, 1,024 x 3,072 x 512 46.5 -> 41.4; Q6_K 1,152 x
+// 6,912 x 203 55.4 -> 47.3; BF16 8,192 x 2,048 x 9 19.8 -> 12.8; F32 2,048 x 2,048
+// x 32 10.9 -> 9.7; only F16 3,072 x 1,024 x 64 (32 x 32) 11.1 -> 11.7.
+// Sixteen waves for the 32 x 32 tile spill (33.5 against 32.2 us and far worse).
+template <uint32_t F, int RB, int TB, uint32_t W, bool FULL, bool CLIP>
+__global__ __launch_bounds__(64 * W, RB == 1 ? 4 : 2) void gemm_exact_short(Product a, uint32_t token_tiles) {
+    constexpr int kSteps = 4;            // groups the inputs are loaded ahead
+    constexpr uint32_t kEach = 32 / W;   // ranges a wave
+    constexpr int kBatch = Codes<F>::kBatch;
+    constexpr int kLoadRows = F == kF32 ? 2 : 1;
+    constexpr uint32_t kBlock = 256 * RB * TB;  // floats of one range's sums
+    constexpr uint32_t kCodeWords = RB * Codes<F>::kWords;
+    constexpr uint32_t kStage = kCodeWords + TB * 512 > kBlock ? kCodeWords + TB * 512 : kBlock;
+    __shared__ float4 sums4[(W - 1) * (kEach - 1) * kBlock / 4];  // the ranges but each wave's last, past wave 0's
+    __shared__ float4 stage4[W * kStage / 4];
+    float* const sums = reinterpret_cast<float*>(sums4);
+    const uint32_t lane = threadIdx.x & 63u, q = lane >> 4, my = lane & 15u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t T = __builtin_amdgcn_readfirstlane(blockIdx.x % token_tiles) * (16 * TB);
+    const uint32_t R = __builtin_amdgcn_readfirstlane(blockIdx.x / token_tiles) * (16 * RB);
     const uint32_t G = a.groups;
-    const uint64_t K = static_cast<uint64_t>(G) * 32;
-    const uint32_t r_begin = 4 * wave;
-    // pair p's steps: its longer range's groups
-    const uint32_t l0 = range_lo(r_begin, G), l1 = range_lo(r_begin + 1, G), l2 = range_lo(r_begin + 2, G),
-                   l3 = range_lo(r_begin + 3, G), l4 = range_lo(r_begin + 4, G);
-    const uint32_t n0 = max(l1 - l0, l2 - l1), steps = n0 + max(l3 - l2, l4 - l3);
-    f32x32 held0 = {}, held1 = {};  // pair 0's sums, pair 1's
+    const auto lo_of = [&](uint32_t r) { return (r * G) >> 5; };  // range_lo; G is below 2^24
+    const uint32_t g_begin = lo_of(kEach * wave), g_end = lo_of(kEach * wave + kEach);
+    float* const stage = reinterpret_cast<float*>(stage4) + wave * kStage;
+    // The stage is this wave's own and its LDS operations run in order, so
+    // ordering the compiler's view of them is all that is needed.
+    auto order = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    f32x4 held[RB][TB];  // the last range's sums; wave 0: its ranges' total
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) held[rb][tb] = f32x4{};
 
-    if (steps) {
+    if (g_begin < g_end) {
+        const uint32_t g_last = g_end - 1;
         // Rows and tokens past the product read its last row or token; their
         // outputs are never stored.
-        const Piece pc = piece_of(a, min(R + (lane & 31u), a.rows - 1));
-        const uint64_t row0 = static_cast<uint64_t>(pc.row) * G;
-        // copy i of a group: token 8 i + lane / 8, its chunk (lane % 8) ^ (token % 8)
-        const float4* src[4];
+        const uint8_t* piece[RB][kLoadRows];
+        uint64_t blocks[RB], row0[RB][kLoadRows];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t tok = 8 * i + (lane >> 3);
-            src[i] = reinterpret_cast<const float4*>(a.x + static_cast<uint64_t>(min(T + tok, a.tokens - 1)) * K) +
-                     ((lane & 7u) ^ (tok & 7u));
-        }
-        const uint32_t my_tok = lane & 31u;
-        float4* const stages = lds + wave * 1024;  // two stages of 2 x 256 chunks, [block][token][chunk]
-        const uint32_t read_at =
-            static_cast<uint32_t>(reinterpret_cast<uintptr_t>(stages)) + 4096 * half + 128 * my_tok;
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int i = 0; i < kLoadRows; ++i) {
+                const Piece pc = piece_of(a, min(R + 16 * rb + 8 * i + Codes<F>::load_row(lane), a.rows - 1));
+                piece[rb][i] = pc.piece, blocks[rb] = pc.blocks, row0[rb][i] = static_cast<uint64_t>(pc.row) * G;
+            }
+        // copy i: token 8 i + lane / 8, its chunk lane % 8 (ks 4c .. 4c + 3)
+        const float4* x[2 * TB];
+        float* const inputs = stage + kCodeWords;
+        uint32_t put_at[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) put_at[e] = operand_word(lane >> 3, lane & 7u, e);
+#pragma unroll
+        for (int i = 0; i < 2 * TB; ++i)
+            x[i] = reinterpret_cast<const float4*>(a.x) + min(T + 8 * i + (lane >> 3), a.tokens - 1) * (G * uint64_t{8}) +
+                   (lane & 7u);
+        const float4* const get_low = reinterpret_cast<const float4*>(inputs) + operand_slot(my, q, 0);
+        const float4* const get_high = reinterpret_cast<const float4*>(inputs) + operand_slot(my, q, 1);
         float lo = 0.0f, hi = 0.0f;
         if constexpr (CLIP) lo = *a.clip[0], hi = *a.clip[1];
-        // Step t's group for block b, clamped into the product; `live` false
-        // past the end of the block's range.
-        auto group_of = [&](uint32_t t, uint32_t b, bool& live) {
-            const bool second = t >= n0;
-            const uint32_t j = second ? t - n0 : t;
-            const uint32_t first = second ? (b ? l3 : l2) : (b ? l1 : l0), end = second ? (b ? l4 : l3) : (b ? l2 : l1);
-            live = first + j < end;
-            return min(first + j, G - 1);
+
+        struct Inputs {
+            float4 v[2 * TB];
         };
-        // A step's copies go out before its weights' loads (and nothing may
-        // move between them), so the wait for its weights covers its copies.
-        auto fetch = [&](Raw<F>& raw, uint32_t stage, uint32_t t) {
-            bool live;
-            const uint32_t g0 = group_of(t, 0, live), g1 = group_of(t, 1, live);
+        auto fetch = [&](Inputs& b, uint32_t g) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                __builtin_amdgcn_global_load_lds(src[i] + 8 * g0, (lds_void)(stages + 512 * stage + 64 * i), 16, 0, 0);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                __builtin_amdgcn_global_load_lds(src[i] + 8 * g1, (lds_void)(stages + 512 * stage + 256 + 64 * i), 16,
-                                                 0, 0);
-            __asm__ __volatile__("" ::: "memory");
-            raw.load(pc.piece, pc.blocks, row0 + (half ? g1 : g0));
+            for (int i = 0; i < 2 * TB; ++i) b.v[i] = x[i][8 * min(g, g_last)];
         };
-        f32x32 s = {};  // +0 at each pair's start: its first products are fma(w, x, +0)
-        auto step = [&](const Raw<F>& raw, uint32_t stage, uint32_t t, auto&& next) {
-            float w[32], x[32];
-            weights_of(raw, w);
-            // the stage's reads, after the weights (whose loads were waited
-            // for): the last weight is an input the reads do not use
-            u32x4s_t q[8];
-            const uint32_t at = read_at + 8192 * stage;
-            const uint32_t sw = my_tok & 7u;
+        auto put = [&](const Inputs& b) {
 #pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const uint32_t addr = at + 16 * (c ^ sw);
-                __asm__ __volatile__("ds_read_b128 %0, %1" : "=v"(q[c]) : "v"(addr), "v"(w[31]));
-            }
-            __asm__ __volatile__("s_waitcnt lgkmcnt(0)"
-                                 : "+v"(q[0]), "+v"(q[1]), "+v"(q[2]), "+v"(q[3]), "+v"(q[4]), "+v"(q[5]),
-                                   "+v"(q[6]), "+v"(q[7]));
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                float4 v = make_float4(__uint_as_float(q[c][0]), __uint_as_float(q[c][1]),
-                                       __uint_as_float(q[c][2]), __uint_as_float(q[c][3]));
+            for (int i = 0; i < 2 * TB; ++i) {
+                float4 v = b.v[i];
                 if constexpr (CLIP) {
-                    v.x = clamp_to(v.x, lo, hi);
-                    v.y = clamp_to(v.y, lo, hi);
-                    v.z = clamp_to(v.z, lo, hi);
-                    v.w = clamp_to(v.w, lo, hi);
+                    v.x = clamp_to(v.x, lo, hi), v.y = clamp_to(v.y, lo, hi);
+                    v.z = clamp_to(v.z, lo, hi), v.w = clamp_to(v.w, lo, hi);
                 }
-                x[4 * c] = v.x;
-                x[4 * c + 1] = v.y;
-                x[4 * c + 2] = v.z;
-                x[4 * c + 3] = v.w;
-            }
-            bool live0, live1;
-            group_of(t, 0, live0);
-            group_of(t, 1, live1);
-            if (!(half ? live1 : live0)) {  // past this block's range: products of -0 and +0
-#pragma unroll
-                for (int k = 0; k < 32; ++k) w[k] = -0.0f, x[k] = 0.0f;
-            }
-            next();  // the next step's loads, in flight under this chain
-#pragma unroll
-            for (int k = 0; k < 32; ++k) s = __builtin_amdgcn_mfma_f32_32x32x1f32(w[k], x[k], s, 0, 0, 0);
-            if (t + 1 == n0) {  // pair 0 ends
-                held0 = s;
-                s = f32x32{};
+                inputs[256 * i + put_at[0]] = v.x;
+                inputs[256 * i + put_at[1]] = v.y;
+                inputs[256 * i + put_at[2]] = v.z;
+                inputs[256 * i + put_at[3]] = v.w;
             }
         };
-        Raw<F> A, B;
-        fetch(A, 0, 0);
-        for (uint32_t t = 0; t < steps; t += 2) {
-            step(A, 0, t, [&] {
-                if (t + 1 < steps) fetch(B, 1, t + 1);
-            });
-            if (t + 1 >= steps) break;
-            step(B, 1, t + 1, [&] {
-                if (t + 2 < steps) fetch(A, 0, t + 2);
-            });
-        }
-        held1 = s;
-    }
-    // Every copy has landed (each wave waited for its last step's weights,
-    // loaded after its copies, and loads nothing past it) and every stage
-    // read: the LDS takes the range sums, [range][register][lane].
-    __syncthreads();
-    float* const sums = reinterpret_cast<float*>(lds);
+        auto fetch_codes = [&](Codes<F> (&c)[RB], uint32_t g) {
 #pragma unroll
-    for (int v = 0; v < 32; ++v) {
-        const uint32_t r = r_begin + (v / 16);
-        sums[r * 1024 + 64 * (v % 16) + lane] = held0[v];
-        sums[(r + 2) * 1024 + 64 * (v % 16) + lane] = held1[v];
-    }
-    __syncthreads();
-
-    // The ordered combine: registers 2 wave and 2 wave + 1 of a block, for `lane`.
-    const uint32_t v0 = 2 * wave;
-    float ta = 0.0f, tb = 0.0f;
-#pragma unroll
-    for (uint32_t r = 0; r < 32; ++r) {
-        if (range_lo(r, G) < range_lo(r + 1, G)) {
-            ta = ta + sums[r * 1024 + 64 * v0 + lane];
-            tb = tb + sums[r * 1024 + 64 * (v0 + 1) + lane];
-        }
-    }
-    const uint32_t token = T + (lane & 31u);
-    const uint32_t p = R + 8 * (v0 / 4) + 4 * (lane >> 5) + (v0 & 3);
-    if (token < a.tokens) {
-        if (p < a.rows) emit<FULL>(a, p, token, token, ta, tb);
-        if (p + 1 < a.rows) emit<FULL>(a, p + 1, token, token, tb, 0.0f);
-    }
-}
-
-// gemm_exact_quad — the short-step tile for a step whose 32 x 32 tiles would
-// leave compute units idle (C6's 2,048 x 8,192 at 32 tokens: 64 of them):
-// 16 rows x 16 tokens a workgroup, four times the workgroups, at twice the
-// decode a product (each instruction does half the products). Each of its
-// eight waves takes four of the 32 ranges as the four blocks of one
-// v_mfma_f32_16x16x1_4b_f32 (K = 1, one fused multiply-add an element): block
-// b is range r_begin + b, its A (row R + l % 16) and B (token T + l % 16) from
-// lanes 16 b .. 16 b + 15, each lane decoding its own range's group; register
-// v holds block v / 4's row 4 (l / 16) + v % 4, column l % 16. Step j is group
-// j of the four ranges; a range a group shorter than the wave's longest takes
-// -0 and +0 at the last step (fma(-0, +0, acc) = acc for every acc). A
-// step's inputs, four groups x 16 tokens x 128 bytes, reach the wave's LDS
-// stage by eight whole-line copies as gemm_exact_short's do, two stages a
-// wave; the accumulator ends as the wave's four range sums, which a barrier
-// later the LDS holds ([range][register][lane]), and 128 threads add a
-// token's rows p, p + 1 over the 32 ranges in order from zero: the bits of
-// every other canonical tile.
-constexpr uint32_t kQuadTile = 16;  // rows, and tokens, a workgroup
-
-template <uint32_t F, bool FULL, bool CLIP>
-__global__ __launch_bounds__(64 * kShortWaves, 1) void gemm_exact_quad(Product a, uint32_t token_tiles) {
-    __shared__ float4 lds[kShortWaves * 2 * 512];  // the stages (16 KB a wave), then the range sums (32 KB)
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6, blk = lane >> 4, my_i = lane & 15u;
-    const uint32_t T = (blockIdx.x % token_tiles) * kQuadTile, R = (blockIdx.x / token_tiles) * kQuadTile;
-    const uint32_t G = a.groups;
-    const uint64_t K = static_cast<uint64_t>(G) * 32;
-    const uint32_t r_begin = 4 * wave;
-    uint32_t lo_r[5];
-#pragma unroll
-    for (int b = 0; b < 5; ++b) lo_r[b] = range_lo(r_begin + b, G);
-    uint32_t steps = 0;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) steps = max(steps, lo_r[b + 1] - lo_r[b]);
-    // this lane's range: its first group and its end
-    const uint32_t my_first = blk == 0 ? lo_r[0] : blk == 1 ? lo_r[1] : blk == 2 ? lo_r[2] : lo_r[3];
-    const uint32_t my_end = blk == 0 ? lo_r[1] : blk == 1 ? lo_r[2] : blk == 2 ? lo_r[3] : lo_r[4];
-    f32x16 s = {};  // +0: each range's first product is fma(w, x, +0)
-
-    if (steps) {
-        // Rows and tokens past the product read its last row or token; their
-        // outputs are never stored.
-        const Piece pc = piece_of(a, min(R + my_i, a.rows - 1));
-        const uint64_t row0 = static_cast<uint64_t>(pc.row) * G;
-        // copy (b, h): block b's tokens 8 h + lane / 8, chunk (lane % 8) ^ (token % 8)
-        const float4* src[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const uint32_t tok = 8 * h + (lane >> 3);
-            src[h] = reinterpret_cast<const float4*>(a.x + static_cast<uint64_t>(min(T + tok, a.tokens - 1)) * K) +
-                     ((lane & 7u) ^ (tok & 7u));
-        }
-        float4* const stages = lds + wave * 1024;  // two stages of 4 x 128 chunks, [block][token][chunk]
-        const uint32_t read_at =
-            static_cast<uint32_t>(reinterpret_cast<uintptr_t>(stages)) + 2048 * blk + 128 * my_i;
-        float lo = 0.0f, hi = 0.0f;
-        if constexpr (CLIP) lo = *a.clip[0], hi = *a.clip[1];
-        // A step's copies go out before its weights' loads (and nothing may
-        // move between them), so the wait for its weights covers its copies.
-        auto fetch = [&](Raw<F>& raw, uint32_t stage, uint32_t j) {
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const uint32_t g = min(lo_r[b] + j, G - 1);
-#pragma unroll
-                for (int h = 0; h < 2; ++h)
-                    __builtin_amdgcn_global_load_lds(src[h] + 8 * g, (lds_void)(stages + 512 * stage + 128 * b + 64 * h),
-                                                     16, 0, 0);
+            for (int rb = 0; rb < RB; ++rb) {
+                if constexpr (F == kF32)
+                    c[rb].load(piece[rb], row0[rb], g, g_last, lane);
+                else
+                    c[rb].load(piece[rb][0], blocks[rb], row0[rb][0], g, g_last, lane);
             }
-            __asm__ __volatile__("" ::: "memory");
-            raw.load(pc.piece, pc.blocks, row0 + min(my_first + j, G - 1));
         };
-        auto step = [&](const Raw<F>& raw, uint32_t stage, uint32_t j, auto&& next) {
-            float w[32], x[32];
-            weights_of(raw, w);
-            // the stage's reads, after the weights (whose loads were waited
-            // for): the last weight is an input the reads do not use
-            u32x4s_t q[8];
-            const uint32_t at = read_at + 8192 * stage;
-            const uint32_t sw = my_i & 7u;
+        // The range being summed and its groups left; below 32 groups the
+        // ranges that hold one hold it alone (group g's is (32 g + 31) / G).
+        uint32_t r = kEach * wave;
+        if (G < 32) r = __builtin_amdgcn_readfirstlane((32 * g_begin + 31) / G);
+        uint32_t left = G < 32 ? 1u : lo_of(r + 1) - lo_of(r);
+        f32x4 s[RB][TB];  // +0 at a range's start: its first product is fma(w, x, +0)
 #pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const uint32_t addr = at + 16 * (c ^ sw);
-                __asm__ __volatile__("ds_read_b128 %0, %1" : "=v"(q[c]) : "v"(addr), "v"(w[31]));
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int tb = 0; tb < TB; ++tb) s[rb][tb] = f32x4{};
+        Inputs buffers[kSteps];
+        constexpr int kCodeBuffers = kSteps / kBatch;
+        Codes<F> codes[kCodeBuffers][RB];
+#pragma unroll
+        for (int i = 0; i < kCodeBuffers; ++i) fetch_codes(codes[i], g_begin + kBatch * i);
+#pragma unroll
+        for (int i = 0; i < kSteps; ++i) fetch(buffers[i], g_begin + i);
+        put(buffers[0]);
+        // Group g, the i-th of four: its codes in the stage or on their way,
+        // its inputs in the stage; `next` holds the next group's.
+        auto step = [&](int i, Inputs& b, const Inputs& next, uint32_t g, bool more) {
+            if (i % kBatch == 0) {
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb) codes[i / kBatch][rb].put(stage + rb * Codes<F>::kWords, lane);
+                if (more) fetch_codes(codes[i / kBatch], g + kSteps);
             }
-            __asm__ __volatile__("s_waitcnt lgkmcnt(0)"
-                                 : "+v"(q[0]), "+v"(q[1]), "+v"(q[2]), "+v"(q[3]), "+v"(q[4]), "+v"(q[5]),
-                                   "+v"(q[6]), "+v"(q[7]));
+            order();
+            float4 bx[TB][2];
 #pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                float4 v = make_float4(__uint_as_float(q[c][0]), __uint_as_float(q[c][1]),
-                                       __uint_as_float(q[c][2]), __uint_as_float(q[c][3]));
-                if constexpr (CLIP) {
-                    v.x = clamp_to(v.x, lo, hi);
-                    v.y = clamp_to(v.y, lo, hi);
-                    v.z = clamp_to(v.z, lo, hi);
-                    v.w = clamp_to(v.w, lo, hi);
+            for (int tb = 0; tb < TB; ++tb) bx[tb][0] = get_low[128 * tb], bx[tb][1] = get_high[128 * tb];
+            Quarter<F> quarter[RB];
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) Codes<F>::get(quarter[rb], stage + rb * Codes<F>::kWords, i % kBatch, lane);
+            order();
+            put(next);
+            if (more) fetch(b, g + kSteps);
+            float w[RB][8];
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) quarter[rb].eight(q, w[rb]);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+#pragma unroll
+                for (int tb = 0; tb < TB; ++tb) {
+                    const float4 h = bx[tb][j / 4];
+                    const float v = j % 4 == 0 ? h.x : j % 4 == 1 ? h.y : j % 4 == 2 ? h.z : h.w;
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb)
+                        s[rb][tb] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[rb][j], v, s[rb][tb], 0, 0, 0);
                 }
-                x[4 * c] = v.x;
-                x[4 * c + 1] = v.y;
-                x[4 * c + 2] = v.z;
-                x[4 * c + 3] = v.w;
             }
-            if (my_first + j >= my_end) {  // past this block's range: products of -0 and +0
+            if (--left == 0) {
+                const uint32_t at = ((kEach - 1) * (wave - 1) + r % kEach) * kBlock + 4 * lane;
 #pragma unroll
-                for (int k = 0; k < 32; ++k) w[k] = -0.0f, x[k] = 0.0f;
+                for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                    for (int tb = 0; tb < TB; ++tb) {
+                        if (wave == 0) {
+                            held[rb][tb] = held[rb][tb] + s[rb][tb];
+                        } else if (r % kEach == kEach - 1) {
+                            held[rb][tb] = s[rb][tb];
+                        } else {
+                            const float e0 = s[rb][tb][0], e1 = s[rb][tb][1], e2 = s[rb][tb][2], e3 = s[rb][tb][3];
+                            *reinterpret_cast<float4*>(sums + at + 256 * (rb * TB + tb)) = make_float4(e0, e1, e2, e3);
+                        }
+                        s[rb][tb] = f32x4{};
+                    }
+                if (G < 32) {
+                    r = __builtin_amdgcn_readfirstlane((32 * (g + 1) + 31) / G);
+                    left = 1;
+                } else {
+                    ++r;
+                    left = lo_of(r + 1) - lo_of(r);
+                }
             }
-            next();  // the next step's loads, in flight under this chain
-#pragma unroll
-            for (int k = 0; k < 32; ++k) s = __builtin_amdgcn_mfma_f32_16x16x1f32(w[k], x[k], s, 0, 0, 0);
         };
-        Raw<F> A, B;
-        fetch(A, 0, 0);
-        for (uint32_t j = 0; j < steps; j += 2) {
-            step(A, 0, j, [&] {
-                if (j + 1 < steps) fetch(B, 1, j + 1);
-            });
-            if (j + 1 >= steps) break;
-            step(B, 1, j + 1, [&] {
-                if (j + 2 < steps) fetch(A, 0, j + 2);
-            });
-        }
-    }
-    // Every copy has landed (each wave waited for its last step's weights,
-    // loaded after its copies, and loads nothing past it) and every stage
-    // read: the LDS takes the range sums, [range][register][lane].
-    __syncthreads();
-    float* const sums = reinterpret_cast<float*>(lds);
+        // The last four groups load nothing more: their loads would be wasted
+        // (a wave of a K = 2,048 product has four or eight groups in all),
+        // and a load that may not be issued would make every wait one for all.
+        uint32_t g = g_begin;
+        for (; g + kSteps < g_end; g += kSteps) {
 #pragma unroll
-    for (int v = 0; v < 16; ++v) sums[(r_begin + v / 4) * 256 + 64 * (v % 4) + lane] = s[v];
+            for (int i = 0; i < kSteps; ++i) step(i, buffers[i], buffers[(i + 1) % kSteps], g + i, true);
+        }
+#pragma unroll
+        for (int i = 0; i < kSteps; ++i)
+            if (g + i < g_end) step(i, buffers[i], buffers[(i + 1) % kSteps], g + i, false);
+    }
+    order();
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+        for (int tb = 0; tb < TB; ++tb) {
+            const float e0 = held[rb][tb][0], e1 = held[rb][tb][1], e2 = held[rb][tb][2], e3 = held[rb][tb][3];
+            *reinterpret_cast<float4*>(stage + 256 * (rb * TB + tb) + 4 * lane) = make_float4(e0, e1, e2, e3);
+        }
     __syncthreads();
 
-    // The ordered combine: registers 2 h and 2 h + 1 of a block, for lane `l`.
-    if (threadIdx.x < 128) {
-        const uint32_t l = threadIdx.x & 63u, h = threadIdx.x >> 6;
-        float ta = 0.0f, tb = 0.0f;
+    // The ordered combine: thread t adds rows 2 h, 2 h + 1 of its lane's four.
+    const uint32_t block = threadIdx.x >> 7, l = threadIdx.x & 63u, h = (threadIdx.x >> 6) & 1u;
+    if (block < RB * TB) {
+        const uint32_t at = 256 * block + 4 * l + 2 * h;
+        const float* const stages = reinterpret_cast<const float*>(stage4);
+        float2 first = *reinterpret_cast<const float2*>(stages + at);
+        float ta = first.x, tb = first.y;
 #pragma unroll
-        for (uint32_t r = 0; r < 32; ++r) {
-            if (range_lo(r, G) < range_lo(r + 1, G)) {
-                ta = ta + sums[r * 256 + 64 * (2 * h) + l];
-                tb = tb + sums[r * 256 + 64 * (2 * h + 1) + l];
+        for (uint32_t r = kEach; r < 32; ++r) {
+            if (lo_of(r) < lo_of(r + 1)) {
+                const float2 v = *reinterpret_cast<const float2*>(
+                    r % kEach == kEach - 1 ? stages + (r / kEach) * kStage + at
+                                           : sums + ((kEach - 1) * (r / kEach - 1) + r % kEach) * kBlock + at);
+                ta = ta + v.x;
+                tb = tb + v.y;
             }
         }
-        const uint32_t token = T + (l & 15u);
-        const uint32_t p = R + 4 * (l >> 4) + 2 * h;
+        const uint32_t token = T + 16 * (block % TB) + (l & 15u);
+        const uint32_t p = R + 16 * (block / TB) + 4 * (l >> 4) + 2 * h;
         if (token < a.tokens) {
             if (p < a.rows) emit<FULL>(a, p, token, token, ta, tb);
             if (p + 1 < a.rows) emit<FULL>(a, p + 1, token, token, tb, 0.0f);
@@ -852,25 +954,25 @@ __global__ __launch_bounds__(64 * kShortWaves, 1) void gemm_exact_quad(Product a
     }
 }
 
+template <uint32_t F, int RB, int TB, uint32_t W>
+void go_short(const Product& a, const Plan& plan, hipStream_t stream) {
+    const dim3 grid(static_cast<uint32_t>(plan.workgroups)), block(64 * W);
+    if (plain_epilogue(a))
+        hipLaunchKernelGGL((gemm_exact_short<F, RB, TB, W, false, false>), grid, block, 0, stream, a, plan.token_tiles);
+    else if (!clipped(a))
+        hipLaunchKernelGGL((gemm_exact_short<F, RB, TB, W, true, false>), grid, block, 0, stream, a, plan.token_tiles);
+    else
+        hipLaunchKernelGGL((gemm_exact_short<F, RB, TB, W, true, true>), grid, block, 0, stream, a, plan.token_tiles);
+}
+
 template <uint32_t F>
 void go_exact_short(const Product& a, const Plan& plan, hipStream_t stream) {
-    const dim3 grid(static_cast<uint32_t>(plan.workgroups)), block(64 * kShortWaves);
-    const uint32_t tt = plan.token_tiles;
-    if (plan.tile_rows == kQuadTile) {
-        if (plain_epilogue(a))
-            hipLaunchKernelGGL((gemm_exact_quad<F, false, false>), grid, block, 0, stream, a, tt);
-        else if (!clipped(a))
-            hipLaunchKernelGGL((gemm_exact_quad<F, true, false>), grid, block, 0, stream, a, tt);
-        else
-            hipLaunchKernelGGL((gemm_exact_quad<F, true, true>), grid, block, 0, stream, a, tt);
-        return;
+    if constexpr (F != kF32) {
+        if (plan.tile_rows == 16 && plan.waves == 16) return go_short<F, 1, 1, 16>(a, plan, stream);
     }
-    if (plain_epilogue(a))
-        hipLaunchKernelGGL((gemm_exact_short<F, false, false>), grid, block, 0, stream, a, tt);
-    else if (!clipped(a))
-        hipLaunchKernelGGL((gemm_exact_short<F, true, false>), grid, block, 0, stream, a, tt);
-    else
-        hipLaunchKernelGGL((gemm_exact_short<F, true, true>), grid, block, 0, stream, a, tt);
+    if (plan.tile_rows == 16) return go_short<F, 1, 1, 8>(a, plan, stream);
+    if (plan.tile_tokens == 16) return go_short<F, 2, 1, 8>(a, plan, stream);
+    go_short<F, 2, 2, 8>(a, plan, stream);
 }
 
 template <uint32_t F, int TB>
@@ -940,16 +1042,22 @@ void plan_gemm_exact_short(const Product& a, uint32_t compute_units, Plan* plan)
     *plan = Plan{};
     plan->kernel = kGemmExactShort;
     plan->launches = 1;
-    // 16 x 16 tiles (gemm_exact_quad) where they number at most two a
-    // compute unit, else 32 x 32 (gemm_exact_short), a quarter as many:
-    // measured on 256 compute units, 2,048 x 2,048 x 32 tokens (256 of 16 x
-    // 16) 7.5 against 17.2 us, 4,096 x 2,048 x 32 (512) 13.6 against 17.8,
-    // 6,144 x 2,048 x 32 (768) 19.8 against 18.0
-    const uint64_t quads = uint64_t{(a.tokens + kQuadTile - 1) / kQuadTile} * ((a.rows + kQuadTile - 1) / kQuadTile);
-    const uint32_t tile = quads <= 2ull * compute_units ? kQuadTile : kShortTile;
-    plan->tile_tokens = tile;
+    // 16 x 16 tiles where they number at most two a compute unit, else 32 x
+    // 32, a quarter as many (16 x 16 against 32 x 32 at three a compute unit:
+    // 6,144 x 2,048 x 32 18.3 against 16.1 us, 6,144 x 4,096 x 32 23.5 against
+    // 26.4); 32 x 16 for steps of at most 16 tokens, whose second 16 would be
+    // padding. Sixteen waves (two ranges each) where the 16 x 16 tiles number
+    // at most one a compute unit and a wave keeps two groups or more: 2,048 x
+    // 8,192 x 32 16.4 against 18.2 us, 2,048 x 2,048 x 16 7.4 against 7.7, but
+    // 1,024 x 1,024 x 64 5.9 against 5.7; F32 always eight (2,048 x 2,048 x 32
+    // 9.7 against 12.1).
+    const uint64_t quads = uint64_t{(a.tokens + 15) / 16} * ((a.rows + 15) / 16);
+    const uint32_t tile = quads <= 2ull * compute_units ? 16 : 32;
+    const uint32_t tile_tokens = a.tokens <= 16 ? 16 : tile;
+    plan->tile_tokens = tile_tokens;
     plan->tile_rows = tile;
-    plan->token_tiles = (a.tokens + tile - 1) / tile;
+    plan->waves = quads <= compute_units && a.groups >= 64 ? 16 : 8;
+    plan->token_tiles = (a.tokens + tile_tokens - 1) / tile_tokens;
     plan->row_tiles = (a.rows + tile - 1) / tile;
     plan->wave_rows = 1;
     plan->wave_tokens = 1;
