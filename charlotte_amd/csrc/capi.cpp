@@ -270,9 +270,20 @@ Verdict plan_product(const chm::Product& a, uint32_t format, const Target& t, ch
         return {};
     }
     if (split) {
-        // the split on the matrix cores' fused multiply-add: the same range
-        // sums, the same combine
-        chm::plan_gemm_exact(a, format, t.compute_units, true, plan);
+        // AUTO, a step of fewer than 32 tokens: the short-step tile, whose
+        // waves split K in the workgroup and add the range sums in LDS, in
+        // one launch (us, against the split and its combine: 2,048 x 2,048 at
+        // 5 / 21 tokens 7.0 / 7.1 against 8.8 / 9.3, 3,072 x 2,048 x 21 10.2
+        // against 13.3, 2,048 x 8,192 x 21 16.3 against 17.3, 4,096 x 14,336 x
+        // 8 25.0 against 39.8) — where its 16 x 16 tiles number more than an
+        // eighth of the compute units: with 32 tiles 512 x 14,336 x 8 takes 24.0
+        // against 22.9. At 32 tokens and more the split stays the plan its
+        // caller's gate asks for (2,048 x 8,192 x 32 18.5 against 16.4).
+        const uint64_t quads = uint64_t{(a.tokens + 15) / 16} * ((a.rows + 15) / 16);
+        if (t.gemm_path == CHARLOTTE_HIP_MATMUL_GEMM_AUTO && a.tokens < 32 && quads > t.compute_units / 8)
+            chm::plan_gemm_exact_short(a, t.compute_units, plan);
+        else  // the split on the matrix cores' fused multiply-add: the same range sums, the same combine
+            chm::plan_gemm_exact(a, format, t.compute_units, true, plan);
         return {};
     }
     chm::Plan exact;

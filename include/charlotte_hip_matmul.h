@@ -121,13 +121,14 @@ typedef enum {
  * step that does not split, AUTO takes the matrix cores' f32
  * instructions (GEMM_EXACT: each range's chain one fused multiply-add a k, as
  * the VALU tile adds it, in 256-row tiles) where the step gives it at least
- * three 64-row, 64- or 32-token shares a compute unit; else the same chains split among a workgroup's
- * waves (GEMM_EXACT_SHORT: 32 rows by 32 tokens, or 16 by 16 where the larger
- * tiles would leave compute units idle, eight waves of four ranges, the range
- * sums combined in LDS). A step that splits runs its chunks of
- * ranges on the matrix-core chains under AUTO and EXACT_MFMA
- * (GEMM_EXACT_SPLIT), on the 128-row VALU tile under CANONICAL (GEMM_SPLIT);
- * the same range sums, the same combine. CANONICAL keeps to the VALU: the
+ * three shares of 64 rows by 64 or 32 tokens a compute unit; else the same
+ * chains split among a workgroup's waves (GEMM_EXACT_SHORT: 32 rows by 32 or
+ * 16 tokens, or 16 by 16 where the larger tiles would leave compute units
+ * idle, the range sums combined in LDS). A step that splits runs its chunks of
+ * ranges on the matrix-core chains under EXACT_MFMA and AUTO
+ * (GEMM_EXACT_SPLIT; AUTO below 32 tokens, but for products of a few rows,
+ * GEMM_EXACT_SHORT, one launch), on the 128-row VALU tile under CANONICAL
+ * (GEMM_SPLIT); the same range sums, the same combine. CANONICAL keeps to the VALU: the
  * 128-row tile, or the short-step tile (GEMM_SHORT: 16 or 8 rows by 32
  * tokens, K split among a workgroup's waves) where the 128-row tiles would
  * number fewer than the compute units. EXACT_MFMA always GEMM_EXACT. All
@@ -320,7 +321,7 @@ typedef enum {
     CHARLOTTE_HIP_MATMUL_KERNEL_GEMM_SHORT = 19,   /* prefill of a short step: 16 or 8 rows x 32 tokens, K split in the workgroup */
     CHARLOTTE_HIP_MATMUL_KERNEL_GEMM_EXACT = 20,   /* prefill on the matrix cores' f32 fused multiply-add, the canonical order */
     CHARLOTTE_HIP_MATMUL_KERNEL_GEMM_EXACT_SPLIT = 21, /* the same split along K, then the ordered combine */
-    CHARLOTTE_HIP_MATMUL_KERNEL_GEMM_EXACT_SHORT = 22  /* a short step on the matrix cores: 32 x 32 or 16 x 16 tiles, K split in the workgroup */
+    CHARLOTTE_HIP_MATMUL_KERNEL_GEMM_EXACT_SHORT = 22  /* a short step on the matrix cores: 32 x 32, 32 x 16 or 16 x 16 tiles, K split in the workgroup */
 } charlotte_hip_matmul_kernel;
 
 /* What a plan is made for: the device's compute units (256 on MI355X) and
