@@ -15,11 +15,12 @@
 // registers once; otherwise the workgroup stages all of x in LDS once,
 // interleaved by range so a half-wave's lanes read consecutive words (L = 32;
 // the two half-waves read the same words: a broadcast).
-// Each step loads all of its groups' bytes before decoding any, so a wave
-// has a step's weights in flight at once.
+// B steps are in flight a wave (gemv_ranges), or a step whole (gemv_quarters),
+// before any is decoded.
 // Range sums meet in LDS, 33 floats a row (padded against bank conflicts);
 // then lane i adds row i's 32 sums in order from zero and writes the output.
 #include <algorithm>
+#include <type_traits>
 
 #include "decode.hpp"
 #include "plan.hpp"
@@ -66,26 +67,92 @@ __device__ __forceinline__ void finish_rows(const Product& a, uint32_t first, ui
 
 // L = 32: lane r of a half-wave owns range r — at most SPAN groups, its
 // chain from zero over them, and no other range; its range sum goes to LDS.
-// Rows a batch: B steps' loads are issued before any is decoded, so a wave
-// keeps B rows' bytes in flight rather than one; B never exceeds a wave's
-// steps, so every row loaded is decoded. The unquantized formats hold 16 or
-// 32 dwords a group, so fewer rows a batch keep the registers in bounds.
+// Steps in flight: B steps' bytes are in registers or on their way, a step's
+// place refilled as soon as it is free; B never exceeds a wave's steps, so
+// every row loaded is decoded. The unquantized formats hold 16 or 32 dwords a
+// group, so fewer steps keep the registers in bounds; two at SPAN 2 leave a
+// third wave a SIMD its registers (Q8_0 128,256 x 2,048, coalesced: 51.2 us at
+// four, 49.4 at two).
 template <uint32_t F>
 constexpr int batch_of(int span) {
     if constexpr (F == kF32) return span >= 2 ? 1 : 2;
     if constexpr (F == kF16 || F == kBF16) return span >= 3 ? 1 : span == 2 ? 2 : 4;
-    return span >= 3 ? 2 : span == 2 ? 4 : 8;
+    return span >= 2 ? 2 : 8;
 }
 
-template <uint32_t F, int SPAN, bool XREG, bool FULL, int B>
+// A lane's slice of its row on the way to it. Slice reads the lane's own
+// bytes: an instruction's lanes are SPAN groups' codes apart, so at 64 bytes
+// and more it touches 32 to 64 lines for 1 KB, and a line has to stay in L1
+// until every instruction that wants 16 of its bytes has run, which with a
+// CU's hundred KB in flight it does not. Chunks (every range SPAN groups
+// exactly, codes of one stream) reads the row's 16-byte chunks in order, 512
+// bytes an instruction a half-wave, non-temporal, and exchanges them through
+// the wave's LDS stage when they are decoded. Chunk e of a lane's N sits there
+// at slot N r + (e xor swizzle(r)), so the lanes that read one chunk index
+// together fall in different banks.
+template <uint32_t F>
+constexpr uint32_t code_bytes() {
+    return F == kF32 ? 128 : F == kF16 || F == kBF16 ? 64 : F == kQ8_0 ? 32 : 16;
+}
+
+template <uint32_t F, int SPAN>
+struct Slice {
+    Raw<F> g[SPAN];
+};
+
+template <uint32_t F, int SPAN>
+struct Chunks {
+    static constexpr uint32_t N = SPAN * code_bytes<F>() / 16;
+    static constexpr uint32_t kPow2 = (N & (0u - N)) < 8 ? (N & (0u - N)) : 8;  // of 2 in N, 8 at most
+    u32x4s_t c[N];
+    uint32_t d[SPAN];
+    static __device__ __forceinline__ uint32_t swizzle(uint32_t r) { return (r / (8 / kPow2)) & (kPow2 - 1); }
+    __device__ __forceinline__ void load(const uint8_t* piece, uint64_t n, uint64_t row0, uint32_t r) {
+        const u32x4s_t* codes = reinterpret_cast<const u32x4s_t*>(piece + code_bytes<F>() * row0);
+#pragma unroll
+        for (uint32_t k = 0; k < N; ++k) {
+            const uint32_t slot = 32 * k + r, to = slot / N;
+            c[k] = __builtin_nontemporal_load(codes + N * to + ((slot % N) ^ swizzle(to)));
+        }
+#pragma unroll
+        for (int i = 0; i < SPAN; ++i) {
+            if constexpr (F == kQ4_1)
+                d[i] = *reinterpret_cast<const uint32_t*>(piece + 16 * n + 4 * (row0 + SPAN * r + i));
+            else if constexpr (!plain_values(F))
+                d[i] = *reinterpret_cast<const uint16_t*>(piece + code_bytes<F>() * n + 2 * (row0 + SPAN * r + i));
+        }
+    }
+    // The half-wave's chunks through its 512 N bytes of stage.
+    __device__ __forceinline__ void exchange(u32x4s_t* stage, uint32_t r, Raw<F> (&raw)[SPAN]) const {
+#pragma unroll
+        for (uint32_t k = 0; k < N; ++k) stage[32 * k + r] = c[k];
+        wave_sync();
+        constexpr uint32_t per = N / SPAN;
+#pragma unroll
+        for (uint32_t e = 0; e < N; ++e) {
+            const u32x4s_t q = stage[N * r + (e ^ swizzle(r))];
+#pragma unroll
+            for (uint32_t w = 0; w < 4; ++w) raw[e / per].w[4 * (e % per) + w] = q[w];
+        }
+        wave_sync();
+#pragma unroll
+        for (int i = 0; i < SPAN; ++i) {
+            if constexpr (F == kQ4_1) raw[i].dm = d[i];
+            else if constexpr (!plain_values(F)) raw[i].d = d[i];
+        }
+    }
+};
+
+template <uint32_t F, int SPAN, bool XREG, bool FULL, int B, bool COALESCED>
 __global__ __launch_bounds__(256, kRangesMinBlocks) void gemv_ranges(Product a, uint32_t steps, uint32_t tiles) {
     // Dynamic LDS: each wave's range sums, then x when it is staged rather
-    // than held in registers. A workgroup is kWaves waves, or one (small
-    // products with x in registers: ranges_waves).
+    // than held in registers, then each wave's exchange stage (coalesced). A
+    // workgroup is kWaves waves, or one (small products with x in registers:
+    // ranges_waves).
     extern __shared__ float4 dynamic_lds[];
     const uint32_t waves_a_block = blockDim.x >> 6;
     float* const partials = reinterpret_cast<float*>(dynamic_lds);
-    float4* const xs4 = dynamic_lds + waves_a_block * (kWaveRows * kRowPad / 4);
+    float4* const xs4 = dynamic_lds + waves_a_block * (steps * 2 * kRowPad / 4);
 
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint32_t half = lane >> 5, r = lane & 31u;
@@ -94,17 +161,23 @@ __global__ __launch_bounds__(256, kRangesMinBlocks) void gemv_ranges(Product a, 
     const uint32_t token = a.last_token ? a.tokens - 1 : 0;
     const float* x = a.x + static_cast<uint64_t>(token) * G * 32;
 
-    Raw<F> raw[B][SPAN];
+    using Held = std::conditional_t<COALESCED, Chunks<F, SPAN>, Slice<F, SPAN>>;
+    Held raw[B];
     // Every lane issues the same loads on every path — rows past the
     // product read its last row, groups past the lane's range the row's last
     // group, unused — so a decode waits for its own loads.
-    auto load_row = [&](Raw<F> (&r)[SPAN], uint32_t wave_first, uint32_t step) {
-        const uint32_t p = min(wave_first + step * 2 + half, a.rows - 1);
+    auto load_row = [&](Held& to, uint32_t first) __attribute__((always_inline)) {
+        const uint32_t p = min(first + half, a.rows - 1);
         const Piece w = piece_of(a, p);
         const uint64_t row0 = static_cast<uint64_t>(w.row) * G;
+        if constexpr (COALESCED) {
+            to.load(w.piece, w.blocks, row0, r);
+        } else {
 #pragma unroll
-        for (int i = 0; i < SPAN; ++i) r[i].load(w.piece, w.blocks, row0 + min(g0 + i, G - 1));
+            for (int i = 0; i < SPAN; ++i) to.g[i].load(w.piece, w.blocks, row0 + min(g0 + i, G - 1));
+        }
     };
+    const uint32_t first_wave_row = (blockIdx.x * waves_a_block + wave) * steps * 2;
     // Staged x: the first tile's first row is issued before x is read and
     // its other rows after, so x's round trip overlaps the weights'. x in
     // registers: x's loads go out first, the rows' behind them — measured
@@ -113,8 +186,7 @@ __global__ __launch_bounds__(256, kRangesMinBlocks) void gemv_ranges(Product a, 
     // row first (x behind it), x coalesced through LDS, or every kernel
     // argument fetched in one batch of scalar loads measured no better. (The
     // grid never exceeds the tiles, so every workgroup has a first tile.)
-    const uint32_t first_wave_row = (blockIdx.x * waves_a_block + wave) * steps * 2;
-    if constexpr (!XREG) load_row(raw[0], first_wave_row, 0);
+    if constexpr (!XREG) load_row(raw[0], first_wave_row);
 
     float xr[XREG ? SPAN * 32 : 1];
     if constexpr (XREG) {
@@ -156,56 +228,81 @@ __global__ __launch_bounds__(256, kRangesMinBlocks) void gemv_ranges(Product a, 
             xs4[256 * k + threadIdx.x] = s0 + k < s1 ? clamp_input(a, xv[k]) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         __syncthreads();
     }
-    if constexpr (XREG) load_row(raw[0], first_wave_row, 0);
+    if constexpr (XREG) load_row(raw[0], first_wave_row);
 #pragma unroll
-    for (int b = 1; b < B; ++b) load_row(raw[b], first_wave_row, b);
+    for (int b = 1; b < B; ++b) load_row(raw[b], first_wave_row + 2 * b);
 
-    float* mine = partials + wave * (kWaveRows * kRowPad);
-    bool loaded = true;  // the first batch already is
-    for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-        const uint32_t wave_first = (tile * waves_a_block + wave) * steps * 2;
-        for (uint32_t step0 = 0; step0 < steps; step0 += B) {
-            if (!loaded) {
+    float* mine = partials + wave * (steps * 2 * kRowPad);
+    u32x4s_t* stage = nullptr;
+    if constexpr (COALESCED)
+        stage = reinterpret_cast<u32x4s_t*>(xs4 + (XREG ? 0 : 256 * SPAN)) + (2 * wave + half) * 32 * Held::N;
+    // The sums of the wave's two rows from `first` — `slot` in its tile.
+    auto decode = [&](const Raw<F> (&raw)[SPAN], uint32_t first, uint32_t slot) __attribute__((always_inline)) {
+        float s = 0.0f;
+        if (first + half < a.rows) {
 #pragma unroll
-                for (int b = 0; b < B; ++b) load_row(raw[b], wave_first, step0 + b);
-            }
-            loaded = false;
+            for (int i = 0; i < SPAN; ++i) {
+                if (COALESCED || g0 + i < g1) {
+                    if constexpr (XREG) {
+                        s = raw[i].chain(xr + 32 * i, s);
+                    } else {
+                        float xg[32];
+                        const float4* src = xs4 + 256 * i + r;
 #pragma unroll
-            for (int b = 0; b < B; ++b) {
-                const uint32_t slot = (step0 + b) * 2 + half;
-                if (step0 + b >= steps) break;
-                float s = 0.0f;
-                if (wave_first + slot < a.rows) {
-#pragma unroll
-                    for (int i = 0; i < SPAN; ++i) {
-                        if (g0 + i < g1) {
-                            if constexpr (XREG) {
-                                s = raw[b][i].chain(xr + 32 * i, s);
-                            } else {
-                                float xg[32];
-                                const float4* src = xs4 + 256 * i + r;
-#pragma unroll
-                                for (int v = 0; v < 8; ++v) {
-                                    const float4 q = src[32 * v];
-                                    xg[4 * v] = q.x;
-                                    xg[4 * v + 1] = q.y;
-                                    xg[4 * v + 2] = q.z;
-                                    xg[4 * v + 3] = q.w;
-                                }
-                                s = raw[b][i].chain(xg, s);
-                            }
+                        for (int v = 0; v < 8; ++v) {
+                            const float4 q = src[32 * v];
+                            xg[4 * v] = q.x;
+                            xg[4 * v + 1] = q.y;
+                            xg[4 * v + 2] = q.z;
+                            xg[4 * v + 3] = q.w;
                         }
+                        s = raw[i].chain(xg, s);
                     }
                 }
-                mine[slot * kRowPad + r] = s;  // an empty range's sum is zero
             }
         }
+        mine[(slot + half) * kRowPad + r] = s;  // an empty range's sum is zero
+    };
+    // B steps in turn, across the tiles' bounds: a step's registers take the
+    // step B on as soon as they are free, so B - 1 to B steps' bytes are in
+    // flight while one decodes (loaded a whole batch at a time and waited for
+    // before the next, direct form: Q4_0 gated 14,336 x 4,096 20.9 -> 18.7 us,
+    // Q8_0 65,536 x 3,072 49.2 -> 45.4). The last B steps load nothing, and a
+    // single batch is all that a small product's wave runs.
+    uint32_t tile = blockIdx.x, step0 = 0, wave_first = first_wave_row;
+    auto batch = [&](auto more, uint32_t next) __attribute__((always_inline)) {
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const uint32_t slot = (step0 + b) * 2;
+            if constexpr (COALESCED) {
+                Raw<F> row[SPAN];
+                raw[b].exchange(stage, r, row);
+                if constexpr (more) load_row(raw[b], next + 2 * b);
+                decode(row, wave_first + slot, slot);
+            } else {
+                decode(raw[b].g, wave_first + slot, slot);
+                if constexpr (more) load_row(raw[b], next + 2 * b);
+            }
+        }
+        if (step0 + B < steps) return;
+        // the tile's last: its rows' totals
         wave_sync();
         float total = 0.0f;
         if (lane < steps * 2 && wave_first + lane < a.rows) total = ordered_total(mine + lane * kRowPad);
         finish_rows<FULL>(a, wave_first, steps * 2, total);
         wave_sync();  // the sums are read before the next tile writes them
+    };
+    while (true) {
+        uint32_t next_tile = tile, next_step = step0 + B, next_first = wave_first;
+        if (next_step >= steps) {
+            next_tile += gridDim.x, next_step = 0;
+            next_first = (next_tile * waves_a_block + wave) * steps * 2;
+        }
+        if (next_tile >= tiles) break;
+        batch(std::true_type{}, next_first + 2 * next_step);
+        tile = next_tile, step0 = next_step, wave_first = next_first;
     }
+    batch(std::false_type{}, 0);
 }
 
 // A lane's run of SPAN groups from gi0. Q4_0 and Q6_K load a run's streams in
@@ -544,22 +641,47 @@ static uint32_t resident(K kernel, size_t lds) {
     return static_cast<uint32_t>(blocks);
 }
 
-template <uint32_t F, int SPAN, bool XREG, bool FULL, int B>
+// Where gemv_ranges reads a product coalesced (K a whole SPAN x 1,024), direct
+// against coalesced, us:
+//   F32 65,536 x 1,024       49.9   44.1    BF16 gated 8,192 x 2,048  18.0   13.5
+//   Q8_0 128,256 x 2,048     54.5   51.2    Q8_0 65,536 x 3,072       45.4   38.6
+// and where it does not: F16 151,936 x 1,024 48.5 against 50.5; Q4_0 gated
+// 14,336 x 4,096 18.7 against 19.6 and Q4_1 65,536 x 2,048 23.6 against 23.5
+// (16 bytes a group: the decode, not the reading, bounds them); F32 and BF16 a
+// group wider and Q8_0 past four groups, whose registers spill.
+constexpr bool ranges_coalesced(uint32_t format, int span) {
+    if (format == kF32) return span == 1;
+    if (format == kF16 || format == kBF16) return span == 2;
+    if (format == kQ8_0) return span >= 2 && span <= 4;
+    return format == kQ4_0 && span == 3;
+}
+
+template <uint32_t F, int SPAN, bool XREG, bool FULL, int B, bool COALESCED>
 static void launch_ranges(const Product& a, uint32_t steps, uint32_t tiles, uint32_t waves, size_t x_lds,
                           uint32_t compute_units, hipStream_t stream) {
-    const size_t lds = waves * kWaveRows * kRowPad * sizeof(float) + x_lds;
+    size_t lds = waves * steps * 2 * kRowPad * sizeof(float) + x_lds;
+    if constexpr (COALESCED) lds += waves * 64 * Chunks<F, SPAN>::N * sizeof(u32x4s_t);
+    const auto kernel = gemv_ranges<F, SPAN, XREG, FULL, B, COALESCED>;
     thread_local size_t cached_lds = ~size_t{0};
     thread_local uint32_t per_cu = 1;
     if (cached_lds != lds) {
         int blocks = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, gemv_ranges<F, SPAN, XREG, FULL, B>, 64 * waves,
-                                                         lds) != hipSuccess ||
-            blocks < 1)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, 64 * waves, lds) != hipSuccess || blocks < 1)
             blocks = 1;
         per_cu = static_cast<uint32_t>(blocks), cached_lds = lds;
     }
     const dim3 grid(std::min(tiles, per_cu * compute_units));
-    hipLaunchKernelGGL((gemv_ranges<F, SPAN, XREG, FULL, B>), grid, dim3(64 * waves), lds, stream, a, steps, tiles);
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), lds, stream, a, steps, tiles);
+}
+
+template <uint32_t F, int SPAN, bool XREG, bool FULL, int B>
+static void pick_ranges(const Product& a, uint32_t steps, uint32_t tiles, uint32_t waves, size_t x_lds,
+                        uint32_t compute_units, hipStream_t stream) {
+    if constexpr (ranges_coalesced(F, SPAN)) {
+        if (a.groups == 32 * SPAN)
+            return launch_ranges<F, SPAN, XREG, FULL, B, true>(a, steps, tiles, waves, x_lds, compute_units, stream);
+    }
+    launch_ranges<F, SPAN, XREG, FULL, B, false>(a, steps, tiles, waves, x_lds, compute_units, stream);
 }
 
 // A grid of at most the workgroups the GPU holds at once, each looping over
@@ -578,15 +700,15 @@ static void go_epilogue(const Product& a, uint32_t steps, uint32_t tiles, uint32
         constexpr uint32_t most = batch_of<F>(SPAN);
         const uint32_t b = std::min(steps, most);
         if (b == 1) {
-            launch_ranges<F, SPAN, XREG, FULL, 1>(a, steps, tiles, waves, lds, compute_units, stream);
+            pick_ranges<F, SPAN, XREG, FULL, 1>(a, steps, tiles, waves, lds, compute_units, stream);
         } else if constexpr (most >= 2) {
             if (b == 2) {
-                launch_ranges<F, SPAN, XREG, FULL, 2>(a, steps, tiles, waves, lds, compute_units, stream);
+                pick_ranges<F, SPAN, XREG, FULL, 2>(a, steps, tiles, waves, lds, compute_units, stream);
             } else if constexpr (most >= 4) {
                 if (b == 4)
-                    launch_ranges<F, SPAN, XREG, FULL, 4>(a, steps, tiles, waves, lds, compute_units, stream);
+                    pick_ranges<F, SPAN, XREG, FULL, 4>(a, steps, tiles, waves, lds, compute_units, stream);
                 else if constexpr (most >= 8)
-                    launch_ranges<F, SPAN, XREG, FULL, 8>(a, steps, tiles, waves, lds, compute_units, stream);
+                    pick_ranges<F, SPAN, XREG, FULL, 8>(a, steps, tiles, waves, lds, compute_units, stream);
             }
         }
     } else {
