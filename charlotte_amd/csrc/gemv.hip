@@ -163,12 +163,25 @@ __global__ __launch_bounds__(256, kRangesMinBlocks) void gemv_ranges(Product a, 
 
     using Held = std::conditional_t<COALESCED, Chunks<F, SPAN>, Slice<F, SPAN>>;
     Held raw[B];
+    // Q6_K with one group a lane: without the members held, the four- and
+    // eight-step loops select a member by its address and wait for all their
+    // loads at each step (us, not held and held: gated 2 x 6,144 x 512 9.4 and
+    // 5.9, 2 x 6,144 x 1,024 9.9 and 6.7, 131,064 x 1,024 28.3 and 25.5). The
+    // other forms do not, and holding them measured up to 5% slower (Q8_0
+    // 131,071 x 512 19.8 against 20.3).
+    Member held[3];
+    const Member* m = a.m;
+    if constexpr (F == kQ6_K && SPAN == 1) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) held[i] = a.m[i], hold(held[i]);
+        m = held;
+    }
     // Every lane issues the same loads on every path — rows past the
     // product read its last row, groups past the lane's range the row's last
     // group, unused — so a decode waits for its own loads.
     auto load_row = [&](Held& to, uint32_t first) __attribute__((always_inline)) {
         const uint32_t p = min(first + half, a.rows - 1);
-        const Piece w = piece_of(a, p);
+        const Piece w = piece_of(a, m, p);
         const uint64_t row0 = static_cast<uint64_t>(w.row) * G;
         if constexpr (COALESCED) {
             to.load(w.piece, w.blocks, row0, r);

@@ -58,16 +58,27 @@ struct Piece {
     uint32_t row;
 };
 
-__device__ __forceinline__ Piece piece_of(const Product& a, uint32_t p) {
+__device__ __forceinline__ Piece piece_of(const Product& a, const Member* m, uint32_t p) {
     if (a.epilogue == kGated) {
         const bool up = p & 1u;
-        return {up ? a.m[1].piece : a.m[0].piece, up ? a.m[1].blocks : a.m[0].blocks,
-                (up ? a.m[1].row_offset : a.m[0].row_offset) + (p >> 1)};
+        return {up ? m[1].piece : m[0].piece, up ? m[1].blocks : m[0].blocks,
+                (up ? m[1].row_offset : m[0].row_offset) + (p >> 1)};
     }
-    Piece w{a.m[0].piece, a.m[0].blocks, a.m[0].row_offset + (p - a.m[0].first)};
-    if (a.members > 1 && p >= a.m[1].first) w = {a.m[1].piece, a.m[1].blocks, a.m[1].row_offset + (p - a.m[1].first)};
-    if (a.members > 2 && p >= a.m[2].first) w = {a.m[2].piece, a.m[2].blocks, a.m[2].row_offset + (p - a.m[2].first)};
+    Piece w{m[0].piece, m[0].blocks, m[0].row_offset + (p - m[0].first)};
+    if (a.members > 1 && p >= m[1].first) w = {m[1].piece, m[1].blocks, m[1].row_offset + (p - m[1].first)};
+    if (a.members > 2 && p >= m[2].first) w = {m[2].piece, m[2].blocks, m[2].row_offset + (p - m[2].first)};
     return w;
+}
+__device__ __forceinline__ Piece piece_of(const Product& a, uint32_t p) { return piece_of(a, a.m, p); }
+
+// The fields piece_of reads, held in scalar registers from here on. Constant
+// indices do not always do it: where loads from the two branches above meet,
+// the compiler may select their addresses instead and load a member's fields
+// a lane from the kernel argument, a wait for every load in flight each time.
+__device__ __forceinline__ void hold(Member& m) {
+    uint64_t piece = reinterpret_cast<uint64_t>(m.piece);
+    __asm__("" : "+s"(piece), "+s"(m.blocks), "+s"(m.row_offset), "+s"(m.first));
+    m.piece = (const uint8_t*)reinterpret_cast<const __attribute__((address_space(1))) uint8_t*>(piece);
 }
 
 // Where product row p's output of `token` goes, and its index o in the

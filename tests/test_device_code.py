@@ -9,6 +9,7 @@ disassembled with the ROCm LLVM tools, and every instruction is checked.
 """
 
 import os
+import re
 import shutil
 import subprocess
 
@@ -59,6 +60,24 @@ def test_no_packed_fp32_instructions(lib, tmp_path):
     assert sum(w.startswith("v_") for w in words) > 100, "too little code disassembled"
     found = {op: words.count(op) for op in PACKED_FP32 if op in words}
     assert not found, f"{os.path.basename(lib)}: packed FP32 instructions {found}"
+
+
+def test_q6_k_decode_loads_nothing_of_its_members_a_lane(tmp_path):
+    """The 32-lane Q6_K decode keeps its members' places in scalar registers.
+    A group is a 16-byte, an 8-byte and two 2-byte loads a lane, and nothing
+    else in a kernel without epilogue options is 4 bytes wide: a 4-byte vector
+    load is a member's row offset, read from the kernel argument between the
+    weights' loads, each with a wait for all of them."""
+    lib = LIBS[0]
+    if not os.path.exists(lib):
+        pytest.skip(f"{os.path.basename(lib)} is not built")
+    kernels = re.split(r"^[0-9a-f]+ <(\S+)>:$", _disassembly(lib, str(tmp_path)), flags=re.M)
+    plain = {n: code for n, code in zip(kernels[1::2], kernels[2::2])
+             if re.search(r"gemv_rangesILj14ELi1ELb1ELb0E", n)}
+    assert len(plain) == 4, sorted(plain)  # one, two, four and eight steps in flight
+    for name, code in plain.items():
+        assert "global_load_dwordx4 " in code and "global_load_ushort " in code
+        assert "global_load_dword " not in code, name
 
 
 def test_the_check_sees_a_packed_instruction(tmp_path):
