@@ -84,12 +84,16 @@ constexpr int batch_of(int span) {
 // bytes: an instruction's lanes are SPAN groups' codes apart, so at 64 bytes
 // and more it touches 32 to 64 lines for 1 KB, and a line has to stay in L1
 // until every instruction that wants 16 of its bytes has run, which with a
-// CU's hundred KB in flight it does not. Chunks (every range SPAN groups
-// exactly, codes of one stream) reads the row's 16-byte chunks in order, 512
-// bytes an instruction a half-wave, non-temporal, and exchanges them through
-// the wave's LDS stage when they are decoded. Chunk e of a lane's N sits there
-// at slot N r + (e xor swizzle(r)), so the lanes that read one chunk index
-// together fall in different banks.
+// CU's hundred KB in flight it does not (F32 33,001 x 1,856 fetched 17% of its
+// lines again; the same loads in another loop, 2%). Chunks reads the row's
+// 16-byte chunks in order, 512 bytes an instruction a half-wave,
+// non-temporal, and exchanges them through the wave's LDS stage when they are
+// decoded. kEven (every range SPAN groups): chunk e of a lane's N lies at slot
+// N r + (e xor swizzle(r)). kUneven (any G): chunk c of the row at place(c).
+// Either way the lanes that read one chunk index together fall in different
+// banks, or two in one.
+enum Read : int { kDirect, kEven, kUneven };
+
 template <uint32_t F>
 constexpr uint32_t code_bytes() {
     return F == kF32 ? 128 : F == kF16 || F == kBF16 ? 64 : F == kQ8_0 ? 32 : 16;
@@ -100,50 +104,62 @@ struct Slice {
     Raw<F> g[SPAN];
 };
 
-template <uint32_t F, int SPAN>
+template <uint32_t F, int SPAN, bool EVEN>
 struct Chunks {
-    static constexpr uint32_t N = SPAN * code_bytes<F>() / 16;
+    static constexpr uint32_t kPer = code_bytes<F>() / 16;  // chunks a group
+    static constexpr uint32_t N = SPAN * kPer;
     static constexpr uint32_t kPow2 = (N & (0u - N)) < 8 ? (N & (0u - N)) : 8;  // of 2 in N, 8 at most
     u32x4s_t c[N];
     uint32_t d[SPAN];
     static __device__ __forceinline__ uint32_t swizzle(uint32_t r) { return (r / (8 / kPow2)) & (kPow2 - 1); }
-    __device__ __forceinline__ void load(const uint8_t* piece, uint64_t n, uint64_t row0, uint32_t r) {
+    static __device__ __forceinline__ uint32_t place(uint32_t chunk) { return chunk ^ (((chunk >> 3) ^ (chunk >> 4)) & 7u); }
+    __device__ __forceinline__ void load(const uint8_t* piece, uint64_t n, uint64_t row0, uint32_t G, uint32_t g0,
+                                         uint32_t r) {
         const u32x4s_t* codes = reinterpret_cast<const u32x4s_t*>(piece + code_bytes<F>() * row0);
 #pragma unroll
         for (uint32_t k = 0; k < N; ++k) {
             const uint32_t slot = 32 * k + r, to = slot / N;
-            c[k] = __builtin_nontemporal_load(codes + N * to + ((slot % N) ^ swizzle(to)));
+            c[k] = __builtin_nontemporal_load(
+                codes + (EVEN ? N * to + ((slot % N) ^ swizzle(to)) : min(slot, kPer * G - 1)));
         }
 #pragma unroll
         for (int i = 0; i < SPAN; ++i) {
+            const uint64_t gi = row0 + (EVEN ? SPAN * r + i : min(g0 + i, G - 1));
             if constexpr (F == kQ4_1)
-                d[i] = *reinterpret_cast<const uint32_t*>(piece + 16 * n + 4 * (row0 + SPAN * r + i));
+                d[i] = *reinterpret_cast<const uint32_t*>(piece + 16 * n + 4 * gi);
             else if constexpr (!plain_values(F))
-                d[i] = *reinterpret_cast<const uint16_t*>(piece + code_bytes<F>() * n + 2 * (row0 + SPAN * r + i));
+                d[i] = *reinterpret_cast<const uint16_t*>(piece + code_bytes<F>() * n + 2 * gi);
         }
     }
-    // The half-wave's chunks through its 512 N bytes of stage.
-    __device__ __forceinline__ void exchange(u32x4s_t* stage, uint32_t r, Raw<F> (&raw)[SPAN]) const {
+    // The half-wave's chunks into its 512 N bytes of stage; the scales pass on
+    // in registers.
+    struct Tails {
+        uint32_t d[SPAN];
+    };
+    __device__ __forceinline__ Tails put(u32x4s_t* stage, uint32_t r) const {
 #pragma unroll
-        for (uint32_t k = 0; k < N; ++k) stage[32 * k + r] = c[k];
-        wave_sync();
-        constexpr uint32_t per = N / SPAN;
+        for (uint32_t k = 0; k < N; ++k) stage[EVEN ? 32 * k + r : place(32 * k + r)] = c[k];
+        Tails t;
 #pragma unroll
-        for (uint32_t e = 0; e < N; ++e) {
-            const u32x4s_t q = stage[N * r + (e ^ swizzle(r))];
+        for (int i = 0; i < SPAN; ++i) t.d[i] = plain_values(F) ? 0 : d[i];
+        return t;
+    }
+    // The lane's group i out of it.
+    static __device__ __forceinline__ Raw<F> get(const u32x4s_t* stage, const Tails& t, uint32_t g0, uint32_t r, int i) {
+        Raw<F> raw;
 #pragma unroll
-            for (uint32_t w = 0; w < 4; ++w) raw[e / per].w[4 * (e % per) + w] = q[w];
+        for (uint32_t e = 0; e < kPer; ++e) {
+            const u32x4s_t q = stage[EVEN ? N * r + ((kPer * i + e) ^ swizzle(r)) : place(kPer * (g0 + i) + e)];
+#pragma unroll
+            for (uint32_t w = 0; w < 4; ++w) raw.w[4 * e + w] = q[w];
         }
-        wave_sync();
-#pragma unroll
-        for (int i = 0; i < SPAN; ++i) {
-            if constexpr (F == kQ4_1) raw[i].dm = d[i];
-            else if constexpr (!plain_values(F)) raw[i].d = d[i];
-        }
+        if constexpr (F == kQ4_1) raw.dm = t.d[i];
+        else if constexpr (!plain_values(F)) raw.d = t.d[i];
+        return raw;
     }
 };
 
-template <uint32_t F, int SPAN, bool XREG, bool FULL, int B, bool COALESCED>
+template <uint32_t F, int SPAN, bool XREG, bool FULL, int B, Read READ>
 __global__ __launch_bounds__(256, kRangesMinBlocks) void gemv_ranges(Product a, uint32_t steps, uint32_t tiles) {
     // Dynamic LDS: each wave's range sums, then x when it is staged rather
     // than held in registers, then each wave's exchange stage (coalesced). A
@@ -161,7 +177,8 @@ __global__ __launch_bounds__(256, kRangesMinBlocks) void gemv_ranges(Product a, 
     const uint32_t token = a.last_token ? a.tokens - 1 : 0;
     const float* x = a.x + static_cast<uint64_t>(token) * G * 32;
 
-    using Held = std::conditional_t<COALESCED, Chunks<F, SPAN>, Slice<F, SPAN>>;
+    constexpr bool COALESCED = READ != kDirect;
+    using Held = std::conditional_t<COALESCED, Chunks<F, SPAN, READ == kEven>, Slice<F, SPAN>>;
     Held raw[B];
     // Q6_K with one group a lane: without the members held, the four- and
     // eight-step loops select a member by its address and wait for all their
@@ -184,7 +201,7 @@ __global__ __launch_bounds__(256, kRangesMinBlocks) void gemv_ranges(Product a, 
         const Piece w = piece_of(a, m, p);
         const uint64_t row0 = static_cast<uint64_t>(w.row) * G;
         if constexpr (COALESCED) {
-            to.load(w.piece, w.blocks, row0, r);
+            to.load(w.piece, w.blocks, row0, G, g0, r);
         } else {
 #pragma unroll
             for (int i = 0; i < SPAN; ++i) to.g[i].load(w.piece, w.blocks, row0 + min(g0 + i, G - 1));
@@ -255,7 +272,7 @@ __global__ __launch_bounds__(256, kRangesMinBlocks) void gemv_ranges(Product a, 
         if (first + half < a.rows) {
 #pragma unroll
             for (int i = 0; i < SPAN; ++i) {
-                if (COALESCED || g0 + i < g1) {
+                if (READ == kEven || g0 + i < g1) {
                     if constexpr (XREG) {
                         s = raw[i].chain(xr + 32 * i, s);
                     } else {
@@ -288,10 +305,30 @@ __global__ __launch_bounds__(256, kRangesMinBlocks) void gemv_ranges(Product a, 
         for (int b = 0; b < B; ++b) {
             const uint32_t slot = (step0 + b) * 2;
             if constexpr (COALESCED) {
-                Raw<F> row[SPAN];
-                raw[b].exchange(stage, r, row);
-                if constexpr (more) load_row(raw[b], next + 2 * b);
-                decode(row, wave_first + slot, slot);
+                // The slice back out whole, where it is at most 32 dwords of
+                // codes (the stage is free sooner), else a group at a time.
+                const typename Held::Tails tails = raw[b].put(stage, r);
+                wave_sync();
+                if constexpr (Held::N <= 8) {
+                    Raw<F> row[SPAN];
+#pragma unroll
+                    for (int i = 0; i < SPAN; ++i) row[i] = Held::get(stage, tails, g0, r, i);
+                    wave_sync();
+                    if constexpr (more) load_row(raw[b], next + 2 * b);
+                    decode(row, wave_first + slot, slot);
+                } else {
+                    if constexpr (more) load_row(raw[b], next + 2 * b);
+                    static_assert(XREG, "the formats with so wide a slice hold x in registers");
+                    float s = 0.0f;
+                    if (wave_first + slot + half < a.rows) {
+#pragma unroll
+                        for (int i = 0; i < SPAN; ++i)
+                            if (READ == kEven || g0 + i < g1)
+                                s = Held::get(stage, tails, g0, r, i).chain(xr + 32 * i, s);
+                    }
+                    mine[(slot + half) * kRowPad + r] = s;
+                    wave_sync();
+                }
             } else {
                 decode(raw[b].g, wave_first + slot, slot);
                 if constexpr (more) load_row(raw[b], next + 2 * b);
@@ -654,27 +691,33 @@ static uint32_t resident(K kernel, size_t lds) {
     return static_cast<uint32_t>(blocks);
 }
 
-// Where gemv_ranges reads a product coalesced (K a whole SPAN x 1,024), direct
-// against coalesced, us:
-//   F32 65,536 x 1,024       49.9   44.1    BF16 gated 8,192 x 2,048  18.0   13.5
-//   Q8_0 128,256 x 2,048     54.5   51.2    Q8_0 65,536 x 3,072       45.4   38.6
-// and where it does not: F16 151,936 x 1,024 48.5 against 50.5; Q4_0 gated
-// 14,336 x 4,096 18.7 against 19.6 and Q4_1 65,536 x 2,048 23.6 against 23.5
-// (16 bytes a group: the decode, not the reading, bounds them); F32 and BF16 a
-// group wider and Q8_0 past four groups, whose registers spill.
-constexpr bool ranges_coalesced(uint32_t format, int span) {
-    if (format == kF32) return span == 1;
-    if (format == kF16 || format == kBF16) return span == 2;
-    if (format == kQ8_0) return span >= 2 && span <= 4;
-    return format == kQ4_0 && span == 3;
+// How gemv_ranges reads a product (`even`: K a whole SPAN x 1,024; `batch`: B),
+// us, direct against coalesced:
+//   F16 131,071 x 1,024  49.4  44.9    BF16 gated 8,192 x 2,048    18.0  13.5
+//   F16 33,001 x 1,856   44.3  29.7    BF16 gated 2 x 6,144 x 2,560 15.3  12.4
+//   F16 33,001 x 3,072   75.1  45.4    F32 65,536 x 1,024          49.9  44.1
+//   F32 33,001 x 1,856   81.0  52.5    F32 gated 2 x 6,144 x 2,048 21.3  17.3
+//   Q8_0 128,256 x 2,048 54.5  51.2    Q8_0 65,536 x 3,072         45.4  38.6
+//   Q8_0 4,096 x 4,096    9.7   8.1    Q4_0 gated 2 x 6,144 x 3,072 14.0  11.8
+// and direct where that is faster: F16 and F32 of uneven ranges of at most a
+// group (33,001 x 512 10.9 against 13.9, and 16.3 against 17.3), F16 and BF16 of
+// uneven ranges of two with one step a wave (1,024 x 1,280 3.05 against 3.20);
+// and, 16 bytes a group, where the decode and not the reading bounds it: Q4_0
+// gated 14,336 x 4,096 18.7 against 19.6, Q4_1 65,536 x 2,048 23.6 against 23.5.
+constexpr Read ranges_read(uint32_t format, int span, int batch, bool even) {
+    const bool halves = format == kF16 || format == kBF16;
+    if (format == kF32) return even ? kEven : span == 2 ? kUneven : kDirect;
+    if (halves) return even ? kEven : span >= 3 || (span == 2 && batch > 1) ? kUneven : kDirect;
+    if (even && ((format == kQ8_0 && span >= 2 && span <= 4) || (format == kQ4_0 && span == 3))) return kEven;
+    return kDirect;
 }
 
-template <uint32_t F, int SPAN, bool XREG, bool FULL, int B, bool COALESCED>
+template <uint32_t F, int SPAN, bool XREG, bool FULL, int B, Read READ>
 static void launch_ranges(const Product& a, uint32_t steps, uint32_t tiles, uint32_t waves, size_t x_lds,
                           uint32_t compute_units, hipStream_t stream) {
     size_t lds = waves * steps * 2 * kRowPad * sizeof(float) + x_lds;
-    if constexpr (COALESCED) lds += waves * 64 * Chunks<F, SPAN>::N * sizeof(u32x4s_t);
-    const auto kernel = gemv_ranges<F, SPAN, XREG, FULL, B, COALESCED>;
+    if constexpr (READ != kDirect) lds += waves * 64 * Chunks<F, SPAN, READ == kEven>::N * sizeof(u32x4s_t);
+    const auto kernel = gemv_ranges<F, SPAN, XREG, FULL, B, READ>;
     thread_local size_t cached_lds = ~size_t{0};
     thread_local uint32_t per_cu = 1;
     if (cached_lds != lds) {
@@ -690,11 +733,12 @@ static void launch_ranges(const Product& a, uint32_t steps, uint32_t tiles, uint
 template <uint32_t F, int SPAN, bool XREG, bool FULL, int B>
 static void pick_ranges(const Product& a, uint32_t steps, uint32_t tiles, uint32_t waves, size_t x_lds,
                         uint32_t compute_units, hipStream_t stream) {
-    if constexpr (ranges_coalesced(F, SPAN)) {
-        if (a.groups == 32 * SPAN)
-            return launch_ranges<F, SPAN, XREG, FULL, B, true>(a, steps, tiles, waves, x_lds, compute_units, stream);
-    }
-    launch_ranges<F, SPAN, XREG, FULL, B, false>(a, steps, tiles, waves, x_lds, compute_units, stream);
+    if (a.groups == 32 * SPAN)
+        launch_ranges<F, SPAN, XREG, FULL, B, ranges_read(F, SPAN, B, true)>(a, steps, tiles, waves, x_lds, compute_units,
+                                                                          stream);
+    else
+        launch_ranges<F, SPAN, XREG, FULL, B, ranges_read(F, SPAN, B, false)>(a, steps, tiles, waves, x_lds,
+                                                                           compute_units, stream);
 }
 
 // A grid of at most the workgroups the GPU holds at once, each looping over
