@@ -72,11 +72,14 @@ __device__ __forceinline__ void finish_rows(const Product& a, uint32_t first, ui
 // every row loaded is decoded. The unquantized formats hold 16 or 32 dwords a
 // group, so fewer steps keep the registers in bounds; two at SPAN 2 leave a
 // third wave a SIMD its registers (Q8_0 128,256 x 2,048, coalesced: 51.2 us at
-// four, 49.4 at two).
+// four, 49.4 at two) — but for Q4_1, which keeps that wave at four (4,099 x
+// 2,048 5.13 us at four, 5.42 at two; gated 2 x 6,144 x 2,048 8.58 and 8.90;
+// 33,001 x 2,048 22.7 and 22.5).
 template <uint32_t F>
 constexpr int batch_of(int span) {
     if constexpr (F == kF32) return span >= 2 ? 1 : 2;
     if constexpr (F == kF16 || F == kBF16) return span >= 3 ? 1 : span == 2 ? 2 : 4;
+    if constexpr (F == kQ4_1) return span >= 3 ? 2 : span == 2 ? 4 : 8;
     return span >= 2 ? 2 : 8;
 }
 
