@@ -25,6 +25,7 @@
 #include "decode.hpp"
 #include "plan.hpp"
 #include "product.hpp"
+#include "resident.hpp"
 #include "stream.hpp"
 
 namespace chm {
@@ -686,11 +687,12 @@ __global__ __launch_bounds__(256, 2) void gemv_chunked(Product a, uint32_t tiles
     }
 }
 
-// Workgroups of `kernel` a CU holds at once with `lds` bytes of dynamic LDS.
+// Workgroups of `threads` of `kernel` a CU holds at once with `lds` bytes of dynamic LDS.
 template <typename K>
-static uint32_t resident(K kernel, size_t lds) {
+static uint32_t resident(K kernel, uint32_t threads, size_t lds) {
     int blocks = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, 256, lds) != hipSuccess || blocks < 1) blocks = 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, threads, lds) != hipSuccess || blocks < 1)
+        blocks = 1;
     return static_cast<uint32_t>(blocks);
 }
 
@@ -721,14 +723,8 @@ static void launch_ranges(const Product& a, uint32_t steps, uint32_t tiles, uint
     size_t lds = waves * steps * 2 * kRowPad * sizeof(float) + x_lds;
     if constexpr (READ != kDirect) lds += waves * 64 * Chunks<F, SPAN, READ == kEven>::N * sizeof(u32x4s_t);
     const auto kernel = gemv_ranges<F, SPAN, XREG, FULL, B, READ>;
-    thread_local size_t cached_lds = ~size_t{0};
-    thread_local uint32_t per_cu = 1;
-    if (cached_lds != lds) {
-        int blocks = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, 64 * waves, lds) != hipSuccess || blocks < 1)
-            blocks = 1;
-        per_cu = static_cast<uint32_t>(blocks), cached_lds = lds;
-    }
+    thread_local ResidentTable table;
+    const uint32_t per_cu = table.of(waves, steps, [&] { return resident(kernel, 64 * waves, lds); });
     const dim3 grid(std::min(tiles, per_cu * compute_units));
     hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), lds, stream, a, steps, tiles);
 }
@@ -774,7 +770,7 @@ static void go_epilogue(const Product& a, uint32_t steps, uint32_t tiles, uint32
     } else {
         thread_local size_t cached_lds = ~size_t{0};
         thread_local uint32_t per_cu = 1;
-        if (cached_lds != lds) per_cu = resident(gemv_quarters<F, SPAN, FULL>, lds), cached_lds = lds;
+        if (cached_lds != lds) per_cu = resident(gemv_quarters<F, SPAN, FULL>, 256, lds), cached_lds = lds;
         const dim3 grid(std::min(tiles, per_cu * compute_units));
         hipLaunchKernelGGL((gemv_quarters<F, SPAN, FULL>), grid, dim3(256), lds, stream, a, steps, tiles);
     }
@@ -794,7 +790,7 @@ static void go_chunked(const Product& a, uint32_t tiles, uint32_t compute_units,
     const bool plain = plain_epilogue(a);
     auto kernel = plain ? gemv_chunked<F, false, STEPS> : gemv_chunked<F, true, STEPS>;
     thread_local uint32_t per_cu[2] = {0, 0};
-    if (per_cu[plain] == 0) per_cu[plain] = resident(kernel, 0);
+    if (per_cu[plain] == 0) per_cu[plain] = resident(kernel, 256, 0);
     const dim3 grid(std::min(tiles, per_cu[plain] * compute_units));
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, stream, a, tiles);
 }
