@@ -267,6 +267,7 @@ Verdict plan_product(const chm::Product& a, uint32_t format, const Target& t, ch
         // the VALU tiles: the short-step tile where the 128-row tiles would
         // be fewer than the compute units
         if (!split && plan->tiles < t.compute_units) chm::plan_gemm_short(a, t.compute_units, plan);
+        plan->gate_splits = split;
         return {};
     }
     if (split) {
@@ -284,6 +285,7 @@ Verdict plan_product(const chm::Product& a, uint32_t format, const Target& t, ch
             chm::plan_gemm_exact_short(a, t.compute_units, plan);
         else  // the split on the matrix cores' fused multiply-add: the same range sums, the same combine
             chm::plan_gemm_exact(a, format, t.compute_units, true, plan);
+        plan->gate_splits = true;
         return {};
     }
     chm::Plan exact;
@@ -590,8 +592,9 @@ charlotte_hip_matmul_status charlotte_hip_matmul_launch(charlotte_hip_matmul_con
     chm::Plan plan;
     if (v.ok()) v = plan_product(a, format, target_of(ctx), gate, range_sums ? range_sums_bytes : 0, &plan);
     if (!v.ok()) return fail(ctx, v.status, v.message);
-    if ((plan.kernel == chm::kGemmSplit || plan.kernel == chm::kGemmExactSplit) &&
-        reinterpret_cast<uintptr_t>(range_sums) % 4 != 0)
+    // Every step that splits by its gate, also where one launch takes it
+    // without range sums: a caller's buffer is refused at any token count.
+    if (plan.gate_splits && reinterpret_cast<uintptr_t>(range_sums) % 4 != 0)
         return fail(ctx, CHARLOTTE_HIP_MATMUL_INVALID_ARGUMENT, "launch: range_sums not 4-byte aligned");
     return run_plan(ctx, a, format, plan, static_cast<float*>(range_sums), stream);
 }

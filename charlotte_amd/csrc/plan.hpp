@@ -38,6 +38,7 @@ struct Plan {
     uint32_t launches = 0;     // kernel launches the product issues
     bool canonical = true;     // the reference's order of addition: bit-exact, batch-invariant
     bool limbs = false;        // decode: the INT8_LIMBS form
+    bool gate_splits = false;  // prefill: the gate and the range sums let the step split, whichever kernel runs it
     bool xreg = false;         // decode (L = 32): x's slice held in registers
     uint32_t lanes = 0;        // decode: lanes a row
     uint32_t span = 0;         // decode: the most groups a lane holds
