@@ -282,7 +282,7 @@ Verdict plan_product(const chm::Product& a, uint32_t format, const Target& t, ch
         // caller's gate asks for (2,048 x 8,192 x 32 18.5 against 16.4).
         const uint64_t quads = uint64_t{(a.tokens + 15) / 16} * ((a.rows + 15) / 16);
         if (t.gemm_path == CHARLOTTE_HIP_MATMUL_GEMM_AUTO && a.tokens < 32 && quads > t.compute_units / 8)
-            chm::plan_gemm_exact_short(a, t.compute_units, plan);
+            chm::plan_gemm_exact_short(a, format, t.compute_units, plan);
         else  // the split on the matrix cores' fused multiply-add: the same range sums, the same combine
             chm::plan_gemm_exact(a, format, t.compute_units, true, plan);
         plan->gate_splits = true;
@@ -302,7 +302,7 @@ Verdict plan_product(const chm::Product& a, uint32_t format, const Target& t, ch
     if (t.gemm_path == CHARLOTTE_HIP_MATMUL_GEMM_EXACT_MFMA || exact_waves >= 3ull * t.compute_units)
         *plan = exact;
     else
-        chm::plan_gemm_exact_short(a, t.compute_units, plan);
+        chm::plan_gemm_exact_short(a, format, t.compute_units, plan);
     return {};
 }
 

@@ -551,24 +551,25 @@ struct Quarter<kF32> {  // the quarter's own eight values
     }
 };
 
-// F16 and BF16: value q of each four, half q % 2 of dword q / 2 of two.
-template <uint32_t F>
-struct QuarterHalves : Raw<F> {
+// BF16: value q of each four, half q % 2 of dword q / 2 of two.
+template <>
+struct Quarter<kBF16> : Raw<kBF16> {
     __device__ __forceinline__ void eight(uint32_t q, float* o) const {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const uint32_t first = this->w[2 * j], second = this->w[2 * j + 1];
-            if constexpr (F == kF16)
-                o[j] = half_to_float(__builtin_amdgcn_perm(second, first, 0x0C0C0100u + 0x0202u * q));
-            else
-                o[j] = __uint_as_float(__builtin_amdgcn_perm(second, first, 0x01000C0Cu + 0x02020000u * q));
-        }
+        for (int j = 0; j < 8; ++j)
+            o[j] = __uint_as_float(__builtin_amdgcn_perm(w[2 * j + 1], w[2 * j], 0x01000C0Cu + 0x02020000u * q));
     }
 };
+
 template <>
-struct Quarter<kF16> : QuarterHalves<kF16> {};
-template <>
-struct Quarter<kBF16> : QuarterHalves<kBF16> {};
+struct Quarter<kF16> {  // the quarter's own eight halves, two a dword
+    uint32_t w[4];
+    __device__ __forceinline__ void eight(uint32_t, float* o) const {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            o[2 * i] = half_to_float(w[i] & 0xFFFFu), o[2 * i + 1] = half_to_float(w[i] >> 16);
+    }
+};
 
 // How sixteen rows' codes reach a wave, kBatch groups at a time: loaded by
 // lanes that read a row's bytes side by side (the four lanes that decode a
@@ -632,27 +633,42 @@ struct Codes {
 };
 
 // F16 and BF16: a group, 64 bytes a row, lane l row l / 4's 16 bytes l % 4.
+// BF16's are read back whole; F16's, whose values each cost a conversion past
+// the pick, are stored [row][quarter][l % 4], a dword the quarter's two values
+// of the eight (4 picks for 8, a lane reads its 16 bytes alone, and 126 registers
+// in place of 136 let two 32 x 16 workgroups on a CU: 6,144 x 1,024 x 100
+// 32.6 -> 32.3 us, 16,384 x 1,024 x 5 12.7 -> 10.8; BF16 so 1-2% slower).
 template <uint32_t F>
 struct HalfCodes {
     static constexpr int kBatch = 1;
     static constexpr uint32_t kWords = 256;
     uint32_t raw[4];
     static __device__ __forceinline__ uint32_t load_row(uint32_t lane) { return lane >> 2; }
+    // 16-byte slot i of a row's four.
+    static __device__ __forceinline__ uint32_t slot(uint32_t row, uint32_t i) { return 4 * row + (i ^ ((row >> 1) & 3u)); }
     __device__ __forceinline__ void load(const uint8_t* piece, uint64_t, uint64_t row0, uint32_t g, uint32_t last,
                                          uint32_t lane) {
         const uint4 c = reinterpret_cast<const uint4*>(piece + 64 * (row0 + min(g, last)))[lane & 3u];
         raw[0] = c.x, raw[1] = c.y, raw[2] = c.z, raw[3] = c.w;
     }
     __device__ __forceinline__ void put(float* stage, uint32_t lane) const {
-        reinterpret_cast<uint4*>(stage)[(lane & ~3u) + ((lane ^ (lane >> 3)) & 3u)] =
-            make_uint4(raw[0], raw[1], raw[2], raw[3]);
+        if constexpr (F == kF16) {
+            uint32_t* const words = reinterpret_cast<uint32_t*>(stage);
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q)  // half q % 2 of dword q / 2 of the first four values, and of the second
+                words[4 * slot(lane >> 2, q) + (lane & 3u)] =
+                    __builtin_amdgcn_perm(raw[2 + q / 2], raw[q / 2], q % 2 ? 0x07060302u : 0x05040100u);
+        } else {
+            reinterpret_cast<uint4*>(stage)[slot(lane >> 2, lane & 3u)] = make_uint4(raw[0], raw[1], raw[2], raw[3]);
+        }
     }
     static __device__ __forceinline__ void get(Quarter<F>& out, const float* stage, uint32_t, uint32_t lane) {
         const uint4* const wide = reinterpret_cast<const uint4*>(stage);
         const uint32_t row = lane & 15u;
+        constexpr uint32_t slots = F == kF16 ? 1 : 4;
 #pragma unroll
-        for (uint32_t i = 0; i < 4; ++i) {
-            const uint4 c = wide[4 * row + (i ^ ((row >> 1) & 3u))];
+        for (uint32_t i = 0; i < slots; ++i) {
+            const uint4 c = wide[slot(row, F == kF16 ? lane >> 4 : i)];
             out.w[4 * i] = c.x, out.w[4 * i + 1] = c.y, out.w[4 * i + 2] = c.z, out.w[4 * i + 3] = c.w;
         }
     }
@@ -1052,7 +1068,7 @@ void plan_gemm_exact(const Product& a, uint32_t format, uint32_t compute_units, 
 }
 
 // The short-step form: workgroups of 32 rows x 32 tokens, token tile first.
-void plan_gemm_exact_short(const Product& a, uint32_t compute_units, Plan* plan) {
+void plan_gemm_exact_short(const Product& a, uint32_t format, uint32_t compute_units, Plan* plan) {
     *plan = Plan{};
     plan->kernel = kGemmExactShort;
     plan->launches = 1;
@@ -1067,7 +1083,15 @@ void plan_gemm_exact_short(const Product& a, uint32_t compute_units, Plan* plan)
     // 9.7 against 12.1).
     const uint64_t quads = uint64_t{(a.tokens + 15) / 16} * ((a.rows + 15) / 16);
     const uint32_t tile = quads <= 2ull * compute_units ? 16 : 32;
-    const uint32_t tile_tokens = a.tokens <= 16 ? 16 : tile;
+    uint32_t tile_tokens = a.tokens <= 16 ? 16 : tile;
+    // F16, and BF16 of K up to 2,048, past two rounds of 32 x 32 tiles: 32 x 16,
+    // of which a CU holds two, one's first loads and combine beside the other's
+    // products (us, 32 x 32 against 32 x 16: F16 6,144 x 1,024 x 100 32.3 and
+    // 29.0, 6,144 x 4,096 x 200 160.6 and 131.9; BF16 gated 2 x 4,096 x 2,048 x
+    // 100 62.9 and 54.1, but 6,144 x 4,096 x 128 78.4 and 81.4).
+    const uint64_t squares = uint64_t{(a.tokens + 31) / 32} * ((a.rows + 31) / 32);
+    if (tile == 32 && (format == kF16 || (format == kBF16 && a.groups <= 64)) && squares > 2ull * compute_units)
+        tile_tokens = 16;
     plan->tile_tokens = tile_tokens;
     plan->tile_rows = tile;
     plan->waves = quads <= compute_units && a.groups >= 64 ? 16 : 8;
