@@ -96,7 +96,8 @@ constexpr int batch_of(int span) {
 // N r + (e xor swizzle(r)). kUneven (any G): chunk c of the row at place(c).
 // Either way the lanes that read one chunk index together fall in different
 // banks, or two in one.
-enum Read : int { kDirect, kEven, kUneven };
+// kBatch: the lane's own bytes, a batch of steps at a time (gemv_ranges).
+enum Read : int { kDirect, kBatch, kEven, kUneven };
 
 template <uint32_t F>
 constexpr uint32_t code_bytes() {
@@ -181,7 +182,7 @@ __global__ __launch_bounds__(256, kRangesMinBlocks) void gemv_ranges(Product a, 
     const uint32_t token = a.last_token ? a.tokens - 1 : 0;
     const float* x = a.x + static_cast<uint64_t>(token) * G * 32;
 
-    constexpr bool COALESCED = READ != kDirect;
+    constexpr bool COALESCED = READ == kEven || READ == kUneven;
     using Held = std::conditional_t<COALESCED, Chunks<F, SPAN, READ == kEven>, Slice<F, SPAN>>;
     Held raw[B];
     // Q6_K with one group a lane: without the members held, the four- and
@@ -335,16 +336,20 @@ __global__ __launch_bounds__(256, kRangesMinBlocks) void gemv_ranges(Product a, 
                 }
             } else {
                 decode(raw[b].g, wave_first + slot, slot);
-                if constexpr (more) load_row(raw[b], next + 2 * b);
+                if constexpr (more && READ == kDirect) load_row(raw[b], next + 2 * b);
             }
         }
-        if (step0 + B < steps) return;
-        // the tile's last: its rows' totals
-        wave_sync();
-        float total = 0.0f;
-        if (lane < steps * 2 && wave_first + lane < a.rows) total = ordered_total(mine + lane * kRowPad);
-        finish_rows<FULL>(a, wave_first, steps * 2, total);
-        wave_sync();  // the sums are read before the next tile writes them
+        if (step0 + B >= steps) {  // the tile's last: its rows' totals
+            wave_sync();
+            float total = 0.0f;
+            if (lane < steps * 2 && wave_first + lane < a.rows) total = ordered_total(mine + lane * kRowPad);
+            finish_rows<FULL>(a, wave_first, steps * 2, total);
+            wave_sync();  // the sums are read before the next tile writes them
+        }
+        if constexpr (more && READ == kBatch) {
+#pragma unroll
+            for (int b = 0; b < B; ++b) load_row(raw[b], next + 2 * b);
+        }
     };
     while (true) {
         uint32_t next_tile = tile, next_step = step0 + B, next_first = wave_first;
@@ -696,32 +701,11 @@ static uint32_t resident(K kernel, uint32_t threads, size_t lds) {
     return static_cast<uint32_t>(blocks);
 }
 
-// How gemv_ranges reads a product (`even`: K a whole SPAN x 1,024; `batch`: B),
-// us, direct against coalesced:
-//   F16 131,071 x 1,024  49.4  44.9    BF16 gated 8,192 x 2,048    18.0  13.5
-//   F16 33,001 x 1,856   44.3  29.7    BF16 gated 2 x 6,144 x 2,560 15.3  12.4
-//   F16 33,001 x 3,072   75.1  45.4    F32 65,536 x 1,024          49.9  44.1
-//   F32 33,001 x 1,856   81.0  52.5    F32 gated 2 x 6,144 x 2,048 21.3  17.3
-//   Q8_0 128,256 x 2,048 54.5  51.2    Q8_0 65,536 x 3,072         45.4  38.6
-//   Q8_0 4,096 x 4,096    9.7   8.1    Q4_0 gated 2 x 6,144 x 3,072 14.0  11.8
-// and direct where that is faster: F16 and F32 of uneven ranges of at most a
-// group (33,001 x 512 10.9 against 13.9, and 16.3 against 17.3), F16 and BF16 of
-// uneven ranges of two with one step a wave (1,024 x 1,280 3.05 against 3.20);
-// and, 16 bytes a group, where the decode and not the reading bounds it: Q4_0
-// gated 14,336 x 4,096 18.7 against 19.6, Q4_1 65,536 x 2,048 23.6 against 23.5.
-constexpr Read ranges_read(uint32_t format, int span, int batch, bool even) {
-    const bool halves = format == kF16 || format == kBF16;
-    if (format == kF32) return even ? kEven : span == 2 ? kUneven : kDirect;
-    if (halves) return even ? kEven : span >= 3 || (span == 2 && batch > 1) ? kUneven : kDirect;
-    if (even && ((format == kQ8_0 && span >= 2 && span <= 4) || (format == kQ4_0 && span == 3))) return kEven;
-    return kDirect;
-}
-
 template <uint32_t F, int SPAN, bool XREG, bool FULL, int B, Read READ>
 static void launch_ranges(const Product& a, uint32_t steps, uint32_t tiles, uint32_t waves, size_t x_lds,
                           uint32_t compute_units, hipStream_t stream) {
     size_t lds = waves * steps * 2 * kRowPad * sizeof(float) + x_lds;
-    if constexpr (READ != kDirect) lds += waves * 64 * Chunks<F, SPAN, READ == kEven>::N * sizeof(u32x4s_t);
+    if constexpr (READ == kEven || READ == kUneven) lds += waves * 64 * Chunks<F, SPAN, READ == kEven>::N * sizeof(u32x4s_t);
     const auto kernel = gemv_ranges<F, SPAN, XREG, FULL, B, READ>;
     thread_local ResidentTable table;
     const uint32_t per_cu = table.of(waves, steps, [&] { return resident(kernel, 64 * waves, lds); });
@@ -729,15 +713,54 @@ static void launch_ranges(const Product& a, uint32_t steps, uint32_t tiles, uint
     hipLaunchKernelGGL(kernel, grid, dim3(64 * waves), lds, stream, a, steps, tiles);
 }
 
+// How gemv_ranges reads a product, by what weights met cold take (rotated over
+// 800 MB), us: a batch at a time / in turn / coalesced. `large`: four waves a
+// workgroup, 2^20 groups or more, so a CU has more than one in flight.
+//   F32     60,001 x 960  41.0 / 50.2 / 35.0    33,001 x 1,920 74.4 / 81.7 / 54.3
+//           gated 2 x 6,912 x 1,920 23.9 / 27.2 / 19.2
+//           in turn up to 20 groups in small products: 4,099 x 512 5.1 / 4.3
+//   F16     78,739 x 1,024 36.9 / 41.2 / 35.2   33,001 x 2,560 64.0 / 66.7 / 39.5
+//           gated 2 x 6,912 x 1,920 15.0 / 20.0 / 11.4
+//           a batch below 24 groups, large: 78,739 x 512 19.1 / 20.6 / 19.5 (read
+//           again at once, from the last-level cache, 15.8 / 17.7 / 18.0)
+//           in turn in small products of up to 48 groups, or uneven threes:
+//           9,001 x 1,280 9.1 / 7.4 / 8.2 (cached 6.5 / 5.7 / 7.7), 4,099 x 2,560
+//           8.5 / 7.9 / 6.9 (5.9 / 5.4 / 6.5)
+//   Q8_0    65,536 x 3,072 49.2 / 45.4 / 38.6   4,096 x 4,096 9.7 / - / 8.1
+//           a batch from 30 groups of one a lane, large: 46,481 x 1,024 13.2 / 14.6
+//           (cached 11.7 / 12.8), but 131,071 x 512 21.3 / 19.3
+//   Q4_0    gated 2 x 6,144 x 3,072 14.0 / - / 11.8; 16 bytes a group are bound by
+//           their decode: gated 14,336 x 4,096 - / 18.7 / 19.6
+// The coalesced form costs weights that are read again from cache at once: F16
+// 78,739 x 1,024 28.9 / 29.5 / 32.6. A model's next step finds few there.
 template <uint32_t F, int SPAN, bool XREG, bool FULL, int B>
 static void pick_ranges(const Product& a, uint32_t steps, uint32_t tiles, uint32_t waves, size_t x_lds,
                         uint32_t compute_units, hipStream_t stream) {
-    if (a.groups == 32 * SPAN)
-        launch_ranges<F, SPAN, XREG, FULL, B, ranges_read(F, SPAN, B, true)>(a, steps, tiles, waves, x_lds, compute_units,
-                                                                          stream);
-    else
-        launch_ranges<F, SPAN, XREG, FULL, B, ranges_read(F, SPAN, B, false)>(a, steps, tiles, waves, x_lds,
-                                                                           compute_units, stream);
+    const auto launch = [&](auto read) {
+        launch_ranges<F, SPAN, XREG, FULL, B, decltype(read)::value>(a, steps, tiles, waves, x_lds, compute_units,
+                                                                     stream);
+    };
+    const bool even = a.groups == 32 * SPAN, large = waves > 1;
+    constexpr bool halves = F == kF16 || F == kBF16;
+    constexpr std::integral_constant<Read, kDirect> direct{};
+    constexpr std::integral_constant<Read, kBatch> batch{};
+    constexpr std::integral_constant<Read, kEven> evenly{};
+    constexpr std::integral_constant<Read, kUneven> unevenly{};
+    if constexpr (F == kF32) {
+        if (even) return launch(evenly);
+        if (SPAN == 2 || large || a.groups > 20) return launch(unevenly);
+    } else if constexpr (halves && SPAN == 1) {
+        if (large && a.groups >= 24) return even ? launch(evenly) : launch(unevenly);
+        if (large) return launch(batch);
+    } else if constexpr (halves) {
+        if (even && (SPAN == 2 || large)) return launch(evenly);
+        if (!even && (large || (SPAN == 2 && a.groups > 48))) return launch(unevenly);
+    } else if constexpr ((F == kQ8_0 && SPAN >= 2 && SPAN <= 4) || (F == kQ4_0 && SPAN == 3)) {
+        if (even) return launch(evenly);
+    } else if constexpr (F == kQ8_0 && SPAN == 1) {
+        if (large && a.groups >= 30) return launch(batch);
+    }
+    launch(direct);
 }
 
 // A grid of at most the workgroups the GPU holds at once, each looping over

@@ -1,14 +1,16 @@
-"""The 32-lane decode's rows read coalesced where a lane's ranges are uneven
-(F32 between K = 1,024 and 2,048, F16 and BF16 between 1,024 and 3,072), and
-its widest even ones (F32 2,048, F16 and BF16 1,024 and 3,072), against the CPU
-oracle bit for bit: ranges of one and two, two and three groups, a group past
-and short of whole; one row, an odd row past a batch's steps; members at odd
-rows, gated pairs and a clip; and more tiles than the grid holds workgroups."""
+"""The 32-lane decode's unquantized rows, by every way of reading them, against
+the CPU oracle bit for bit: coalesced where a lane's ranges are uneven (F32
+past 20 groups, F16 and BF16 past 48 and in large products), and in the widest
+even ones (F32 2,048, F16 and BF16 1,024 and 3,072), a batch at a time (large F16,
+BF16 and Q8_0 products) and in turn: ranges of none and one, one and two, two
+and three groups, a group past and short of whole; one row, an odd row past a
+batch's steps; members at odd rows, gated pairs and a clip; and more tiles than
+the grid holds workgroups."""
 
 import numpy as np
 import pytest
 
-from tests.support.oracle_lib import BF16, F16, F32
+from tests.support.oracle_lib import BF16, F16, F32, Q8_0
 
 pytestmark = pytest.mark.gpu
 THREADS = 16
@@ -24,17 +26,19 @@ def run():
     c.close()
 
 
-CASES = [(F32, 1056), (F32, 1504), (F32, 2016), (F32, 2048), (F16, 1024), (F16, 1056), (F16, 1856), (F16, 2016),
+CASES = [(F32, 640), (F32, 704), (F32, 992), (F16, 640), (F16, 992), (BF16, 992), (Q8_0, 960), (F32, 1056), (F32, 1504), (F32, 2016), (F32, 2048), (F16, 1024), (F16, 1056), (F16, 1856), (F16, 2016),
          (F16, 2080), (F16, 2560), (F16, 3040), (F16, 3072), (BF16, 1024), (BF16, 1504), (BF16, 2080), (BF16, 3072)]
 
 
 @pytest.mark.parametrize("gtype,columns", CASES)
-@pytest.mark.parametrize("rows", [1, 67, 2051, 20003])
+@pytest.mark.parametrize("rows", [1, 67, 2051, 20003, 53003])
 def test_rows_of_every_remainder_are_the_oracles_bits(oracle, run, gtype, columns, rows):
     from charlotte_amd import matmul as mm
     from charlotte_amd import synthetic
     from tests.support.gpu import bits_equal, first_difference
 
+    if rows * columns > 53003 * 1056:
+        rows = 53003 * 1056 // columns | 1  # the oracle's time; 2^20 groups and more all the same
     rng = np.random.default_rng(rows + columns)
     stored = synthetic.weight(rng, int(gtype), rows, columns)
     x = synthetic.activations(rng, 1, columns)
@@ -46,7 +50,7 @@ def test_rows_of_every_remainder_are_the_oracles_bits(oracle, run, gtype, column
     assert bits_equal(got, want), first_difference(got, want)
 
 
-@pytest.mark.parametrize("gtype,columns", [(F32, 1504), (F32, 2048), (F16, 1856), (F16, 2560), (BF16, 3072)])
+@pytest.mark.parametrize("gtype,columns", [(F32, 800), (F32, 1504), (F32, 2048), (F16, 1856), (F16, 2560), (BF16, 3072)])
 def test_members_and_gated_pairs(oracle, run, gtype, columns):
     from charlotte_amd import matmul as mm
     from charlotte_amd import synthetic
@@ -74,7 +78,7 @@ def test_members_and_gated_pairs(oracle, run, gtype, columns):
         w.free()
 
 
-@pytest.mark.parametrize("gtype,columns", [(F32, 1056), (F16, 1056), (BF16, 2080)])
+@pytest.mark.parametrize("gtype,columns", [(F32, 800), (F32, 1056), (F16, 640), (F16, 992), (F16, 1056), (BF16, 2080), (Q8_0, 992)])
 def test_a_workgroup_of_several_tiles(oracle, run, gtype, columns):
     """140,001 rows, a 4,099-row weight over and over: 64-row tiles, four and
     more for each workgroup of the at most 768 that 256 compute units hold."""
