@@ -1051,6 +1051,7 @@ void plan_gemm_exact(const Product& a, uint32_t format, uint32_t compute_units, 
     plan->launches = split ? 2 : 1;
     plan->tile_tokens = tt;
     plan->tile_rows = kWaves * kWaveRows;
+    plan->waves = kWaves;
     plan->token_tiles = (a.tokens + tt - 1) / tt;
     plan->row_tiles = (a.rows + plan->tile_rows - 1) / plan->tile_rows;
     plan->wave_rows = kWaveRows / 32;
@@ -1067,7 +1068,8 @@ void plan_gemm_exact(const Product& a, uint32_t format, uint32_t compute_units, 
     plan->workgroups = plan->tiles * chunks;
 }
 
-// The short-step form: workgroups of 32 rows x 32 tokens, token tile first.
+// The short-step form: workgroups of 32 rows x 32 or 16 tokens, or 16 x 16,
+// token tile first.
 void plan_gemm_exact_short(const Product& a, uint32_t format, uint32_t compute_units, Plan* plan) {
     *plan = Plan{};
     plan->kernel = kGemmExactShort;
@@ -1094,7 +1096,7 @@ void plan_gemm_exact_short(const Product& a, uint32_t format, uint32_t compute_u
         tile_tokens = 16;
     plan->tile_tokens = tile_tokens;
     plan->tile_rows = tile;
-    plan->waves = quads <= compute_units && a.groups >= 64 ? 16 : 8;
+    plan->waves = format != kF32 && quads <= compute_units && a.groups >= 64 ? 16 : 8;
     plan->token_tiles = (a.tokens + tile_tokens - 1) / tile_tokens;
     plan->row_tiles = (a.rows + tile - 1) / tile;
     plan->wave_rows = 1;

@@ -30,7 +30,7 @@ enum Kernel : uint32_t {
     kGemmShort = 19,    // prefill of a short step: 16 or 8 rows x 32 tokens, K split among the waves
     kGemmExact = 20,    // prefill on the matrix cores' f32 instructions, the canonical order
     kGemmExactSplit = 21,  // the same split along K, then the ordered combine
-    kGemmExactShort = 22,  // a short step on the matrix cores: 32 x 32, K split among 8 waves
+    kGemmExactShort = 22,  // a short step on the matrix cores: 32 x 32, 32 x 16 or 16 x 16, K split among 8 or 16 waves
 };
 
 struct Plan {
@@ -43,7 +43,7 @@ struct Plan {
     uint32_t lanes = 0;        // decode: lanes a row
     uint32_t span = 0;         // decode: the most groups a lane holds
     uint32_t steps = 0;        // decode: steps a wave
-    uint32_t waves = 4;        // decode (L = 32): waves a workgroup, 4 or 1
+    uint32_t waves = 4;        // waves a workgroup (decode, L = 32: 4 or 1; the exact tiles: 8 or 16)
     uint32_t tile_tokens = 0;  // prefill: tokens a workgroup's tile (decode: 1)
     uint32_t tile_rows = 0;    // product rows a workgroup's tile
     uint32_t token_tiles = 0, row_tiles = 0;
