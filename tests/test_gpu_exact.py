@@ -1,15 +1,15 @@
 """The matrix-core prefill in the canonical order (GEMM_EXACT) against the
 128-row VALU tile, bit for bit, at full size.
 
-GEMM_EXACT runs each range's chain on v_mfma_f32_32x32x1_2b_f32, one fused
-multiply-add a k, so its outputs are the VALU tile's bits whatever the
-inputs. The oracle holds both tiles to the reference order at small sizes
+GEMM_EXACT runs each range's chain on v_mfma_f32_32x32x2_f32, two fused
+multiply-adds an instruction in k order, so its outputs are the VALU tile's
+bits whatever the inputs. The oracle holds both tiles to the reference order at small sizes
 (test_gpu_parity, _formats, _float_formats, _epilogues and _edges run under
 EXACT_MFMA too); here the two tiles meet where the oracle would take too long:
 the BASELINE prefill shapes in full (C4; C5's QKV, gated gate/up and down at
 2,048 tokens), Q6_K products, K past the ranges' count (K = 14,336) and
 below it (K = 64: 30 empty ranges), ragged rows and tokens, every epilogue,
-on both of its tiles (64 tokens a wave for large steps, 32 for the rest);
+on both of its tiles (64 tokens a workgroup for large steps, 32 for the rest);
 and its split along K (GEMM_EXACT_SPLIT) against the VALU's (GEMM_SPLIT).
 The reference's own check of the same property: a token's outputs the same
 whatever the step (tests/gpu/matmul_test.cpp:257-267).
@@ -258,10 +258,9 @@ def short_ctxs():
     (Q8_0, 8192, 64, 32, 32),    # 2 groups: pairs with an empty range
 ])
 def test_short_step_tile_same_bits_as_the_valu_short_tile(short_ctxs, gtype, rows, columns, tokens, tile):
-    """GEMM_EXACT_SHORT against the VALU short-step tile, bit for bit: 32 x 32
-    tiles (each wave four of the ranges, two a 32x32x1 two-block instruction)
-    where they give every compute unit one, else 16 x 16 (four ranges a
-    16x16x1 four-block instruction); the sums combined in LDS."""
+    """GEMM_EXACT_SHORT against the VALU short-step tile, bit for bit: 16 x 16
+    tiles where they number at most two a compute unit, else 32 x 32; each
+    wave's ranges on the K = 4 instruction, the sums combined in LDS."""
     from charlotte_amd import matmul as mm
     from charlotte_amd import synthetic
 
@@ -286,9 +285,8 @@ def test_short_step_tile_same_bits_as_the_valu_short_tile(short_ctxs, gtype, row
 @pytest.mark.parametrize("rows,tile", [(640, 16), (12288, 32)])
 def test_short_step_tile_special_inputs_as_the_valu_short_tile(short_ctxs, rows, tile):
     """Infinite, NaN, huge, subnormal and signed-zero inputs through ranges of
-    unequal length (45 groups, a shorter range multiplying -0 by +0 at its
-    last step), on both tile sizes: NaN where the VALU short tile has NaN,
-    every other output bit for bit."""
+    unequal length (45 groups), on 16 x 16 and 32 x 16 tiles (5 tokens): NaN
+    where the VALU short tile has NaN, every other output bit for bit."""
     from charlotte_amd import matmul as mm
     from charlotte_amd import synthetic
 

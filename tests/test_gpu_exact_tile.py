@@ -37,15 +37,20 @@ def _run(ctx, gtype, parts, columns, x, widths, offsets=None, **kw):
 
 
 @pytest.mark.parametrize("gtype", [Q4_0, Q4_1, Q8_0, Q6_K, F32, F16, BF16])
-@pytest.mark.parametrize("rows,columns,tokens", [(264, 544, 31), (504, 1056, 33), (16392, 96, 1025)])
+@pytest.mark.parametrize("rows,columns,tokens", [(264, 544, 31), (504, 1056, 33), (16392, 96, 1025),
+                                                 (16328, 96, 1001)])
 def test_edges_same_bits_as_the_tile(ctxs, gtype, rows, columns, tokens):
-    """(16,392 rows x 1,025 tokens take 64-token tiles, the others 32.)"""
+    """(16,328 rows x 1,001 tokens take 64-token tiles, but in F32, the others 32.)"""
+    from charlotte_amd import matmul as mm
     from charlotte_amd import synthetic
     from tests.support.gpu import bits_equal, first_difference
 
     rng = np.random.default_rng(rows + columns + tokens)
     stored = synthetic.weight(rng, int(gtype), rows, columns)
     x = synthetic.activations(rng, tokens, columns)
+    shape = mm.MatmulLaunch([mm.Member(mm.Weight.shape(gtype, rows, columns))], 16, [16])
+    p = mm.plan_launch(shape, tokens, mm.Target(256, mm.GemmPath.EXACT_MFMA))
+    assert p.tile_tokens == (64 if tokens == 1001 and gtype != F32 else 32)
     got, want = (_run(c, gtype, [(rows, stored)], columns, x, [rows])[0] for c in ctxs)
     assert bits_equal(got, want), first_difference(got, want)
 

@@ -1,8 +1,9 @@
-"""The matrix-core instruction the canonical-order prefill tiles (GEMM_EXACT,
-GEMM_EXACT_SHORT, GEMM_EXACT_SPLIT) are built on, v_mfma_f32_32x32x1_2b_f32,
-and its four-block K = 1 sibling v_mfma_f32_16x16x1_4b_f32 are, element by
-element, one fused multiply-add, d = fmaf(a, b, c), bit for bit; and their
-lane layouts.
+"""The f32 matrix-core instructions are, element by element, fused
+multiply-adds in k order, bit for bit; and their lane layouts. The canonical-
+order prefill tiles are built on two of them: v_mfma_f32_32x32x2_f32
+(GEMM_EXACT, GEMM_EXACT_SPLIT) and v_mfma_f32_16x16x4_f32 (GEMM_EXACT_SHORT). The
+K = 1 shapes, v_mfma_f32_32x32x1_2b_f32 and v_mfma_f32_16x16x1_4b_f32, show
+the single step: d = fmaf(a, b, c).
 
 GEMM_EXACT's outputs are the reference order's bits only because of that, so
 the property itself is held here, on the harness's probes (harness.hip):
@@ -131,7 +132,7 @@ def test_accumulators_come_back_in_their_places(shape, registers):
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape", [5, 6])
 def test_k1_f32_instruction_layout(shape):
-    """The places the exact prefill tiles read results from. 32x32x1 (two
+    """The places results come back in. 32x32x1 (two
     blocks, 32 registers): register v of lane l is block v / 16, its row 8
     ((v % 16) / 4) + 4 (l / 32) + v % 4 (a from lane 32 (v / 16) + that row),
     its column l % 32 (b from lane 32 (v / 16) + l % 32). 16x16x1 (four
