@@ -273,15 +273,19 @@ Verdict plan_product(const chm::Product& a, uint32_t format, const Target& t, ch
     if (split) {
         // AUTO, a step of fewer than 32 tokens: the short-step tile, whose
         // waves split K in the workgroup and add the range sums in LDS, in
-        // one launch (us, against the split and its combine: 2,048 x 2,048 at
-        // 5 / 21 tokens 7.0 / 7.1 against 8.8 / 9.3, 3,072 x 2,048 x 21 10.2
-        // against 13.3, 2,048 x 8,192 x 21 16.3 against 17.3, 4,096 x 14,336 x
-        // 8 25.0 against 39.8) — where its 16 x 16 tiles number more than an
-        // eighth of the compute units: with 32 tiles 512 x 14,336 x 8 takes 24.0
-        // against 22.9. At 32 tokens and more the split stays the plan its
-        // caller's gate asks for (2,048 x 8,192 x 32 18.5 against 16.4).
+        // one launch (us, Q4_0, against the split and its combine: 2,048 x 2,048
+        // at 16 / 31 tokens 6.2 / 6.3 against 8.4 / 9.2, 3,072 x 2,048 x 31 9.6
+        // against 13.9, 2,048 x 8,192 x 31 15.7 against 16.4, 4,096 x 14,336 x
+        // 16 25.2 against 40.2) — where its 16 x 16 tiles number more than an
+        // eighth of the compute units (with 32 tiles 512 x 14,336 x 16 takes
+        // 23.2 against 22.0), and past 16 tokens where K is at most 8,192: beyond,
+        // each wave's own walk through K is the time (4,096 x 14,336 x 31 46.6
+        // against 43.0, BF16 51.6 against 43.0). From 32 tokens the split stays
+        // the plan its caller's gate asks for, the short tile by now the faster
+        // at 32 on all but the longest rows (2,048 x 8,192 15.7 against 16.4).
         const uint64_t quads = uint64_t{(a.tokens + 15) / 16} * ((a.rows + 15) / 16);
-        if (t.gemm_path == CHARLOTTE_HIP_MATMUL_GEMM_AUTO && a.tokens < 32 && quads > t.compute_units / 8)
+        if (t.gemm_path == CHARLOTTE_HIP_MATMUL_GEMM_AUTO && a.tokens < 32 && quads > t.compute_units / 8 &&
+            (a.tokens <= 16 || a.groups <= 256))
             chm::plan_gemm_exact_short(a, format, t.compute_units, plan);
         else  // the split on the matrix cores' fused multiply-add: the same range sums, the same combine
             chm::plan_gemm_exact(a, format, t.compute_units, true, plan);
@@ -291,13 +295,14 @@ Verdict plan_product(const chm::Product& a, uint32_t format, const Target& t, ch
     chm::Plan exact;
     chm::plan_gemm_exact(a, format, t.compute_units, false, &exact);
     // AUTO: the matrix cores' fused multiply-add tile where the step gives it
-    // at least three waves a compute unit (at fewer each of its waves' walk
-    // through K is the step's time: measured slower than the short-step tile
-    // at 640 waves on 256 compute units, 91 against 79 us at 2,560 x 2,048 x
-    // 512 tokens, faster at 768, 53 against 58 us at 3,072 x 1,024 x 512);
-    // else the short-step form on the matrix cores, K split among a
-    // workgroup's waves (measured faster than the VALU short-step tile at
-    // every short step tried). The same bits whichever runs.
+    // at least three shares of 64 rows by its tokens a compute unit (at fewer
+    // each workgroup's walk through K is the step's time: slower than the
+    // short-step tile at 640 shares on 256 compute units, 80 against 73 us at
+    // 2,560 x 2,048 x 512 tokens, faster at 768, 43 against 55 at 3,072 x 1,024 x
+    // 512; with K about 1,024 already a little below, 43 against 45 at 4,096 x
+    // 1,024 x 300's 640); else the short-step form on the matrix cores, K split
+    // among a workgroup's waves (measured faster than the VALU short-step tile
+    // at every short step tried). The same bits whichever runs.
     const uint64_t exact_waves = uint64_t{(a.rows + 63) / 64} * exact.token_tiles;
     if (t.gemm_path == CHARLOTTE_HIP_MATMUL_GEMM_EXACT_MFMA || exact_waves >= 3ull * t.compute_units)
         *plan = exact;

@@ -126,10 +126,10 @@ typedef enum {
  * 16 tokens, or 16 by 16 where the larger tiles would leave compute units
  * idle, the range sums combined in LDS). A step that splits runs its chunks of
  * ranges on the matrix-core chains under EXACT_MFMA and AUTO
- * (GEMM_EXACT_SPLIT; AUTO below 32 tokens, but for products of a few rows,
- * GEMM_EXACT_SHORT, one launch), on the 128-row VALU tile under CANONICAL
- * (GEMM_SPLIT); the same range sums, the same combine. CANONICAL keeps to the VALU: the
- * 128-row tile, or the short-step tile (GEMM_SHORT: 16 or 8 rows by 32
+ * (GEMM_EXACT_SPLIT; AUTO below 32 tokens, but for products of a few rows and,
+ * past 16 tokens, of K past 8,192, GEMM_EXACT_SHORT, one launch), on the 128-row
+ * VALU tile under CANONICAL (GEMM_SPLIT); the same range sums, the same
+ * combine. CANONICAL keeps to the VALU: the 128-row tile, or the short-step tile (GEMM_SHORT: 16 or 8 rows by 32
  * tokens, K split among a workgroup's waves) where the 128-row tiles would
  * number fewer than the compute units. EXACT_MFMA always GEMM_EXACT. All
  * three give the same bits.

@@ -1,7 +1,7 @@
 """AUTO's plan for a step its gate would split: below 32 tokens the short-step
 tile in one launch, where its 16 x 16 tiles number more than an eighth of the
-compute units; from 32 tokens, for fewer tiles, and under EXACT_MFMA and
-CANONICAL, the split."""
+compute units, and past 16 tokens where K is at most 8,192; from 32 tokens, for
+fewer tiles or longer rows, and under EXACT_MFMA and CANONICAL, the split."""
 
 import pytest
 
@@ -29,3 +29,14 @@ def test_the_plan_of_a_step_the_gate_splits(rows, tokens, path, kernel):
     # without the gate, or without range sums, nothing splits
     for kw in ({"gate": mm.kNever, "range_sums_bytes": 1 << 30}, {"gate": mm.kAlways, "range_sums_bytes": 0}):
         assert mm.plan_launch(m, tokens, mm.Target(256, path), **kw).launches == 1
+
+
+@pytest.mark.parametrize("columns,tokens,kernel", [
+    (8192, 31, K.GEMM_EXACT_SHORT), (8224, 17, K.GEMM_EXACT_SPLIT), (14336, 16, K.GEMM_EXACT_SHORT),
+    (14336, 17, K.GEMM_EXACT_SPLIT), (14336, 31, K.GEMM_EXACT_SPLIT),
+])
+def test_long_rows_past_sixteen_tokens_split(columns, tokens, kernel):
+    w = mm.Weight.shape(Q4_0, 4096, columns)
+    p = mm.plan_launch(mm.MatmulLaunch([mm.Member(w)], 16, [16]), tokens, mm.Target(256), gate=mm.kAlways,
+                       range_sums_bytes=1 << 30)
+    assert p.kernel == kernel
