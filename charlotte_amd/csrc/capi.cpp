@@ -299,8 +299,8 @@ Verdict plan_product(const chm::Product& a, uint32_t format, const Target& t, ch
     // each workgroup's walk through K is the step's time: slower than the
     // short-step tile at 640 shares on 256 compute units, 80 against 73 us at
     // 2,560 x 2,048 x 512 tokens, faster at 768, 43 against 55 at 3,072 x 1,024 x
-    // 512; with K about 1,024 already a little below, 43 against 45 at 4,096 x
-    // 1,024 x 300's 640); else the short-step form on the matrix cores, K split
+    // 512; already a little below, 81 against 87 at 6,144 x 2,048 x 200's 672 and
+    // 43 against 45 at 4,096 x 1,024 x 300's 640); else the short-step form on the matrix cores, K split
     // among a workgroup's waves (measured faster than the VALU short-step tile
     // at every short step tried). The same bits whichever runs.
     const uint64_t exact_waves = uint64_t{(a.rows + 63) / 64} * exact.token_tiles;

@@ -750,11 +750,11 @@ struct Codes<kF32> {
 // launch, the first loads' round trip and the combine. Measured against the
 // K = 1 forms (a pair of ranges, or four, the blocks of one instruction, two
 // groups' inputs staged by LDS copies), us: Q4_0 16,384 x 2,048 at 5 tokens
-// 33.6 -> 16.8, 8,192 x 2,048 at 16 / 64 14.0 -> 11.2 / 34.6 -> 32.2, 2,048 x
-// 8,192 at 5 / 32 19.7 -> 15.9 / 20.5 -> 16.4, 4,096 x 2,048 x 32 13.6 -> 10.5,
-// 2,048 x 2,048 x 32 7.4 -> 7.1, 1,024 x 3,072 x 512 46.5 -> 41.4; Q6_K 1,152 x
-// 6,912 x 203 55.4 -> 47.3; BF16 8,192 x 2,048 x 9 19.8 -> 12.8; F32 2,048 x 2,048
-// x 32 10.9 -> 9.7; only F16 3,072 x 1,024 x 64 (32 x 32) 11.1 -> 11.7.
+// 32.3 -> 15.6, 8,192 x 2,048 at 16 / 64 13.2 -> 9.7 / 33.2 -> 30.0, 2,048 x
+// 8,192 at 5 / 32 18.7 -> 14.8 / 19.3 -> 15.2, 4,096 x 2,048 x 32 13.2 -> 9.7,
+// 2,048 x 2,048 x 32 7.2 -> 6.3, 1,024 x 3,072 x 512 45.2 -> 40.1; Q6_K 1,152 x
+// 6,912 x 203 54.6 -> 46.0; BF16 8,192 x 2,048 x 9 16.2 -> 10.2; F32 2,048 x 2,048
+// x 32 11.0 -> 9.0; F16 3,072 x 1,024 x 64 (32 x 32) 11.3 -> 10.4.
 // Sixteen waves for the 32 x 32 tile spill (33.5 against 32.2 us and far worse).
 template <uint32_t F, int RB, int TB, uint32_t W, bool FULL, bool CLIP>
 __global__ __launch_bounds__(64 * W, RB == 1 ? 4 : 2) void gemm_exact_short(Product a, uint32_t token_tiles) {

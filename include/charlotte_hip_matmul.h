@@ -129,10 +129,10 @@ typedef enum {
  * (GEMM_EXACT_SPLIT; AUTO below 32 tokens, but for products of a few rows and,
  * past 16 tokens, of K past 8,192, GEMM_EXACT_SHORT, one launch), on the 128-row
  * VALU tile under CANONICAL (GEMM_SPLIT); the same range sums, the same
- * combine. CANONICAL keeps to the VALU: the 128-row tile, or the short-step tile (GEMM_SHORT: 16 or 8 rows by 32
- * tokens, K split among a workgroup's waves) where the 128-row tiles would
- * number fewer than the compute units. EXACT_MFMA always GEMM_EXACT. All
- * three give the same bits.
+ * combine. CANONICAL keeps to the VALU: the 128-row tile, or the short-step
+ * tile (GEMM_SHORT: 16 or 8 rows by 32 tokens, K split among a workgroup's
+ * waves) where the 128-row tiles would number fewer than the compute units.
+ * EXACT_MFMA always GEMM_EXACT. All three give the same bits.
  * SPLIT_F16_MFMA, only when asked for, runs the products on the matrix cores
  * with x split into two f16 parts, within the tolerance max|err| / max|y| <=
  * 1e-5 but not bit-exact and not batch-invariant with decode; it needs a
